@@ -190,7 +190,8 @@ int ifx_dequant_rows(const void* x, int x_dtype, int64_t ldx, int64_t M, int64_t
  * 16-byte aligned device memory, used when the GEMM (M > 64) splits K across
  * workgroups because it has too few output tiles to fill the GPU: the slices'
  * fp32 partial sums, added by a second launch. The size is 0 (NULL allowed)
- * otherwise, and always for M <= 64. No initialisation is needed; one
+ * otherwise, and always for M <= 64. With K % 128 != 0 a smaller workspace (or
+ * NULL) is accepted too: K is then not split. No initialisation is needed; one
  * workspace serves any sequence of calls and shapes. Calls that may overlap
  * must not share a workspace.
  * With sa = sw = NULL and epilogue 0 this is the raw-accumulator GEMM of
@@ -329,7 +330,9 @@ int ifx_wan_qkv(const void* raw, int raw_dtype, int64_t ldraw, const float* row,
  * launches, the output bit-identical to those two calls in sequence.
  * IFX_SCALE_TENSOR needs ldx == K (else IFX_ERR_UNSUPPORTED).
  * workspace: ifx_quant_linear_workspace_size(...) bytes, 256-byte aligned, no
- * initialisation needed; calls that may overlap must not share one.
+ * initialisation needed; calls that may overlap must not share one. With
+ * K % 128 != 0 the part of ifx_fp8_linear_workspace_size may be missing (K is
+ * then not split).
  * a_scale: NULL, or [M] f32 (IFX_SCALE_ROW) / [1] f32 (IFX_SCALE_TENSOR) that
  * receives the activation scales. IFX_EPI_SCALAR_SA is rejected (the scale is
  * computed here); IFX_EPI_SCALAR_SW is honoured.
@@ -417,7 +420,8 @@ int ifx_attention(const void* q, const void* k, const void* v, void* o, int dtyp
  * (ifx_quant_linear_noalloc_max_bytes() = 64 MiB per GPU, held from the first
  * call on that GPU until the process ends). No allocation of any kind.
  * Rejects with IFX_ERR_SCRATCH a call whose ifx_quant_linear_workspace_size
- * exceeds the scratch (about M * K bytes of e4m3 plus the split-K partials).
+ * exceeds the scratch (about M * K bytes of e4m3 plus the split-K partials;
+ * with K % 128 != 0 a call whose partials do not fit runs without a split).
  * The scratch is looked up on the CURRENT device (hipGetDevice), which must be
  * the device of `stream` and of every operand. All calls on one GPU share its
  * scratch: calls that may overlap on one GPU (distinct streams without

@@ -22,19 +22,17 @@
 // unchanged.
 //
 // Kernels (dispatch in ifx_fp8_linear)
-//  * gemm_big (M > 64, K % 128 == 0): 256 weight rows x 256 (or fewer) tokens
+//  * gemm_big (M > 64): 256 weight rows x 256 (or fewer) tokens
 //    per workgroup, 32x32x64 MFMAs, operands copied global -> LDS by
 //    direct-to-LDS DMA through a multi-stage ring, LDS-staged epilogue; split K
 //    (+ splitk_reduce) when the output has too few tiles to fill the GPU.
-//  * gemm_lds (M > 64 with K % 128 != 0): BN x BM tile, 16x16x128 MFMAs,
-//    register-staged double-buffered LDS tiles (16-byte chunks XOR-swizzled by
-//    row), epilogue from registers.
 //  * gemm_skinny (M <= 64): bound by the weight stream. A workgroup owns 16 (32
 //    for GLU) weight rows and the whole of K; its waves split the K steps,
 //    stream weight fragments straight from HBM into MFMA registers, and add
 //    their partial sums in LDS in a fixed order (deterministic).
 
 #include <algorithm>
+#include <iterator>
 #include <mutex>
 #include <type_traits>
 
@@ -173,14 +171,6 @@ __device__ __forceinline__ float4 load_res4(const Epi& e, int64_t m, int64_t c) 
                      __uint_as_float(r.y & 0xFFFF0000u));
 }
 
-// Plain epilogue for one lane's D fragment: rows n..n+3 of W, token m.
-__device__ __forceinline__ void epi_store(const Epi& e, const v4f acc, int64_t n, int64_t m) {
-  if (m >= e.M || n >= e.N) return;
-  float y[4];
-  epi_pre(e, acc, n, m, y);
-  epi_finish4(e, m, n, y);
-}
-
 // GLU first half: `ng` is the packed row of the gate fragment, the up fragment
 // is 16 packed rows later. Caller guarantees m < M, ng < N.
 __device__ __forceinline__ void epi_pre_glu(const Epi& e, const v4f accg, const v4f accu, int64_t ng,
@@ -200,15 +190,6 @@ __device__ __forceinline__ void epi_pre_glu(const Epi& e, const v4f accg, const 
   for (int r = 0; r < 4; ++r) y[r] = (swiglu ? silu(g[r]) : gelu_tanh(g[r])) * u[r];
 }
 
-// GLU epilogue; output column = (ng / 32) * 16 + (ng % 16).
-__device__ __forceinline__ void epi_store_glu(const Epi& e, const v4f accg, const v4f accu, int64_t ng,
-                                              int64_t m) {
-  if (m >= e.M || ng >= e.N) return;
-  float y[4];
-  epi_pre_glu(e, accg, accu, ng, m, y);
-  epi_finish4(e, m, (ng >> 5) * 16 + (ng & 15), y);
-}
-
 __device__ __forceinline__ v4f mfma16(const v8i& w, const v8i& a, const v4f& c) {
   // cbsz = blgp = 0: both operands are FP8 E4M3 (OCP); no block scales.
   return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(w, a, c, 0, 0, 0, 0, 0, 0);
@@ -224,155 +205,7 @@ __device__ __forceinline__ v4i ld16_nt(const uint8_t* p) {
   return __builtin_nontemporal_load(reinterpret_cast<const v4i*>(p));
 }
 
-// ---------------------------------------------------------------------------
-// Large-M kernel: LDS double-buffered tiles
-// ---------------------------------------------------------------------------
-
-constexpr int kBK = 128;  // K bytes per stage (one MFMA K step)
-
-template <int BN, int BM, int WGN, int WGM, bool GLU>
-struct TileCfg {
-  static constexpr int kThreads = WGN * WGM * 64;
-  static constexpr int kTN = BN / WGN;  // wave tile (weight rows)
-  static constexpr int kTM = BM / WGM;  // wave tile (tokens)
-  static constexpr int kFN = kTN / 16;
-  static constexpr int kFM = kTM / 16;
-  static constexpr int kCW = BN * 8 / kThreads;  // 16-byte chunks per thread per stage
-  static constexpr int kCA = BM * 8 / kThreads;
-  static constexpr int kStageBytes = (BN + BM) * kBK;
-  static_assert(kTN % 16 == 0 && kTM % 16 == 0, "wave tile");
-  static_assert(!GLU || kFN % 2 == 0, "GLU needs gate/up fragment pairs");
-  static_assert(BN * 8 % kThreads == 0 && BM * 8 % kThreads == 0, "load split");
-  static_assert(2 * kStageBytes <= 160 * 1024, "LDS");
-};
-
-// Byte offset of 16-byte chunk `ch` of tile row `row` (rows are 128 bytes).
-// gfx950's LDS serves a ds_read_b128 16 lanes at a time from 64 banks (a
-// 256-byte window = two tile rows). A fragment read has 16 lanes on 16
-// consecutive rows with the same logical chunk, so the physical chunk
-// ch ^ f(row), f(row) = (row % 8) ^ ((row / 8) % 2), must put every
-// (row parity, chunk) pair in a different place: f is a bijection on the even
-// and on the odd rows of any 16-row block (and on any 8 consecutive rows,
-// which also keeps a 32-bank, 8-lanes-per-cycle LDS conflict free).
-__device__ __forceinline__ int swz_f(int row) { return (row & 7) ^ ((row >> 3) & 1); }
-__device__ __forceinline__ int swz(int row, int ch) { return row * kBK + ((ch ^ swz_f(row)) << 4); }
-
-template <int BN, int BM, int WGN, int WGM, bool GLU>
-__global__ __launch_bounds__(WGN* WGM * 64, 1) void gemm_lds(const uint8_t* __restrict__ A, int64_t lda,
-                                                             const uint8_t* __restrict__ W, int64_t ldw,
-                                                             int64_t K, int tiles_m, Epi e) {
-  using C = TileCfg<BN, BM, WGN, WGM, GLU>;
-  __shared__ __attribute__((aligned(16))) uint8_t smem[2 * C::kStageBytes];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int wn = wave / WGM;
-  const int wm = wave % WGM;
-
-  // Tile order: consecutive workgroups walk M first, sharing one weight tile.
-  const int tm = blockIdx.x % tiles_m;
-  const int tn = blockIdx.x / tiles_m;
-  const int64_t n0 = static_cast<int64_t>(tn) * BN;
-  const int64_t m0 = static_cast<int64_t>(tm) * BM;
-  const int nk = static_cast<int>((K + kBK - 1) / kBK);
-
-  // Per-thread global chunk coordinates (fixed across stages).
-  const uint8_t* wsrc[C::kCW];
-  int wdst[C::kCW];
-#pragma unroll
-  for (int i = 0; i < C::kCW; ++i) {
-    const int c = tid + i * C::kThreads;
-    const int row = c >> 3, ch = c & 7;
-    int64_t n = n0 + row;
-    n = n < e.N ? n : e.N - 1;  // clamp: rows past N are computed but never stored
-    wsrc[i] = W + n * ldw + ch * 16;
-    wdst[i] = swz(row, ch);
-  }
-  const uint8_t* asrc[C::kCA];
-  int adst[C::kCA];
-#pragma unroll
-  for (int i = 0; i < C::kCA; ++i) {
-    const int c = tid + i * C::kThreads;
-    const int row = c >> 3, ch = c & 7;
-    int64_t m = m0 + row;
-    m = m < e.M ? m : e.M - 1;
-    asrc[i] = A + m * lda + ch * 16;
-    adst[i] = BN * kBK + swz(row, ch);
-  }
-
-  uint4 pw[C::kCW], pa[C::kCA];
-  auto gload = [&](int kt) {
-    const int64_t k0 = static_cast<int64_t>(kt) * kBK;
-#pragma unroll
-    for (int i = 0; i < C::kCW; ++i) {
-      const int ch = (tid + i * C::kThreads) & 7;
-      pw[i] = (k0 + ch * 16 < K) ? *reinterpret_cast<const uint4*>(wsrc[i] + k0) : make_uint4(0, 0, 0, 0);
-    }
-#pragma unroll
-    for (int i = 0; i < C::kCA; ++i) {
-      const int ch = (tid + i * C::kThreads) & 7;
-      pa[i] = (k0 + ch * 16 < K) ? *reinterpret_cast<const uint4*>(asrc[i] + k0) : make_uint4(0, 0, 0, 0);
-    }
-  };
-  auto sstore = [&](int buf) {
-    uint8_t* base = smem + buf * C::kStageBytes;
-#pragma unroll
-    for (int i = 0; i < C::kCW; ++i) *reinterpret_cast<uint4*>(base + wdst[i]) = pw[i];
-#pragma unroll
-    for (int i = 0; i < C::kCA; ++i) *reinterpret_cast<uint4*>(base + adst[i]) = pa[i];
-  };
-
-  v4f acc[C::kFN][C::kFM];
-#pragma unroll
-  for (int i = 0; i < C::kFN; ++i)
-#pragma unroll
-    for (int j = 0; j < C::kFM; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
-
-  // Fragment read offsets: lane supplies row lane%16, chunks 2g and 2g+1.
-  const int frow = lane & 15;
-  const int g = lane >> 4;
-
-  gload(0);
-  sstore(0);
-  __syncthreads();
-  for (int kt = 0; kt < nk; ++kt) {
-    const int buf = kt & 1;
-    if (kt + 1 < nk) gload(kt + 1);
-    const uint8_t* base = smem + buf * C::kStageBytes;
-    v8i af[C::kFM];
-#pragma unroll
-    for (int j = 0; j < C::kFM; ++j) {
-      const int row = wm * C::kTM + j * 16 + frow;
-      const uint8_t* p = base + BN * kBK;
-      af[j] = cat8(ld16(p + swz(row, 2 * g)), ld16(p + swz(row, 2 * g + 1)));
-    }
-#pragma unroll
-    for (int i = 0; i < C::kFN; ++i) {
-      const int row = wn * C::kTN + i * 16 + frow;
-      const v8i wf = cat8(ld16(base + swz(row, 2 * g)), ld16(base + swz(row, 2 * g + 1)));
-#pragma unroll
-      for (int j = 0; j < C::kFM; ++j) acc[i][j] = mfma16(wf, af[j], acc[i][j]);
-    }
-    if (kt + 1 < nk) sstore(buf ^ 1);
-    __syncthreads();
-  }
-
-  // Epilogue straight from the accumulators.
-  const int64_t nb = n0 + wn * C::kTN + 4 * g;
-  const int64_t mb = m0 + wm * C::kTM + frow;
-  if constexpr (GLU) {
-#pragma unroll
-    for (int i = 0; i < C::kFN; i += 2)
-#pragma unroll
-      for (int j = 0; j < C::kFM; ++j) epi_store_glu(e, acc[i][j], acc[i + 1][j], nb + i * 16, mb + j * 16);
-  } else {
-#pragma unroll
-    for (int i = 0; i < C::kFN; ++i)
-#pragma unroll
-      for (int j = 0; j < C::kFM; ++j) epi_store(e, acc[i][j], nb + i * 16, mb + j * 16);
-  }
-}
+constexpr int kBK = 128;  // K bytes of a skinny K step and of a large-M stage (one 16x16x128 MFMA)
 
 // ---------------------------------------------------------------------------
 // Large-M kernel: direct-to-LDS multi-stage ring, 32x32x64 matrix cores
@@ -393,7 +226,15 @@ __global__ __launch_bounds__(WGN* WGM * 64, 1) void gemm_lds(const uint8_t* __re
 // instruction moves 64 lanes x 16 B into a contiguous 1 KB LDS block, lane l
 // landing at byte 16*l; the row swizzle (`Swz`) is therefore applied on the
 // global side, each lane fetching the logical chunk that belongs at its LDS
-// position. K must be a multiple of KB (whole stages, no zero fill).
+// position.
+//
+// K that is no multiple of KB: stage 0 holds the K % KB bytes at the end of the
+// rows (each lane whose chunk lies past K fetches 16 zero bytes instead), and
+// stage t >= 1 the bytes from (t - 1) * KB on. The partial stage comes first
+// because its per-lane addresses then stay in the prologue, which also issues
+// it early: the K loop is the same code for every K (against register-staged
+// tiles without the ring: 768x1152x4304 25.0 -> 16.9 us, 8000x4112x3088 234 ->
+// 110, 1000x14016x2000 GeGLU 86 -> 37, 200x3008x8208 55.7 -> 20.7).
 //
 // OCC workgroups share a CU (OCC = 2 with 64-byte stages: 3 x 24 KB of LDS and
 // <= 128 VGPRs per wave), so one workgroup's barrier waits, epilogue and store
@@ -488,6 +329,9 @@ __device__ __forceinline__ v4f quad(const v16f& v, int q) {
   return v4f{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
 }
 
+// What a DMA lane fetches for a chunk past K.
+__device__ const uint8_t kZeroChunk[16] __attribute__((aligned(16))) = {};
+
 template <int BM, int BN, int KB, int STAGES, int OCC, bool GLU, int FM>
 __global__ __launch_bounds__(4 * BM / FM, OCC) void gemm_big(const uint8_t* __restrict__ A, int64_t lda,
                                                      const uint8_t* __restrict__ W, int64_t ldw, int64_t K,
@@ -534,9 +378,13 @@ __global__ __launch_bounds__(4 * BM / FM, OCC) void gemm_big(const uint8_t* __re
   if (!map_tile(tmap, tm, tn, split)) return;
   const int64_t n0 = static_cast<int64_t>(tn) * BN;
   const int64_t m0 = static_cast<int64_t>(tm) * BM;
-  // this workgroup's K stages: [kt0, kt0 + nk)
+  // this workgroup's K stages: [kt0, kt0 + nk); with a partial stage (number
+  // 0, `tail` bytes) stage t >= 1 starts at byte t * KB - kshift
   const int kt0 = static_cast<int>(split * part.kstages);
-  const int nk = static_cast<int>(min(static_cast<int64_t>(K / KB) - kt0, part.kstages));
+  const int nk = static_cast<int>(min((K + KB - 1) / KB - kt0, part.kstages));
+  const int tail = static_cast<int>(K % KB);
+  const int kshift = tail ? KB : 0;
+  const bool tail_here = tail && kt0 == 0;
 
   // Epilogue operands of this lane (column scales, bias, adaLN gate) and this
   // thread's token scale, loaded before the K loop so their latency hides
@@ -573,20 +421,25 @@ __global__ __launch_bounds__(4 * BM / FM, OCC) void gemm_big(const uint8_t* __re
   const int lpos = lane % S::kChunks;
   const uint32_t lds_base = __builtin_amdgcn_readfirstlane(lds_offset(smem) + wave * kLoads * 1024);
   const int64_t n_last = e.N - 1, m_last = e.M - 1;
-  auto issue = [&](int kl) {  // local stage index kl: K stage kt0 + kl, ring slot kl % STAGES
-    const int kt = kt0 + kl;
+  // Issues this wave's DMAs of local stage kl (K stage kt0 + kl) into ring slot
+  // kl % STAGES; with the tag, of the partial stage, whose chunks past K come
+  // from zeros.
+  auto issue = [&](int kl, auto tail_tag) {
+    constexpr bool kTail = decltype(tail_tag)::value;
     const uint32_t buf = lds_base + (kl % STAGES) * kStage;
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) {
       const int blk = wave * kLoads + i;
       const int row = blk * kRowsPerDma + lrow;
-      const int64_t k0 = static_cast<int64_t>(kt) * KB + ((lpos ^ S::f(row)) << 4);
+      const int kb = (lpos ^ S::f(row)) << 4;
+      const int64_t k0 = (kTail ? K - tail : static_cast<int64_t>(kt0 + kl) * KB - kshift) + kb;
       const uint8_t* p;
       if (blk * kRowsPerDma < BN) {  // wave-uniform
         p = W + min(n0 + row, n_last) * ldw + k0;
       } else {
         p = A + min(m0 + (row - BN), m_last) * lda + k0;
       }
+      if constexpr (kTail) p = kb < tail ? p : kZeroChunk;
       dma16(p, buf + i * 1024);
     }
   };
@@ -654,7 +507,7 @@ __global__ __launch_bounds__(4 * BM / FM, OCC) void gemm_big(const uint8_t* __re
     constexpr int kW4 = BN / 32, kA4 = BM / 32;  // kW3: weight / token DMAs per wave per stage
     static_assert(!kW3 || kW4 + kA4 == kLoads, "kW3 DMA split");
     const int iw = kW3 ? kW4 : BN / 8 - wave * kLoads;  // DMAs i < iw of this wave load weight rows
-    uint32_t doff[kLoads];                  // per-lane byte offset of DMA i, stage kt0
+    uint32_t doff[kLoads];  // per-lane byte offset of DMA i, stage kt0 (modulo 2^32; whole stages only)
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) {
       const int blk = kW3 ? (i < kW4 ? wave * kW4 + i : BN / 8 + wave * kA4 + (i - kW4)) : wave * kLoads + i;
@@ -662,7 +515,7 @@ __global__ __launch_bounds__(4 * BM / FM, OCC) void gemm_big(const uint8_t* __re
       const bool isw = i < iw;
       const uint32_t row = static_cast<uint32_t>(isw ? min(n0 + r, n_last) : min(m0 + (r - BN), m_last));
       doff[i] = __umul24(row, static_cast<uint32_t>(isw ? ldw : lda)) +
-                static_cast<uint32_t>(((lpos ^ lrow ^ (blk & 1)) << 4) + kt0 * KB);
+                static_cast<uint32_t>(((lpos ^ lrow ^ (blk & 1)) << 4) + kt0 * KB - kshift);
     }
     const uint64_t wbase = reinterpret_cast<uintptr_t>(W), abase = reinterpret_cast<uintptr_t>(A);
     // LDS byte offsets (from smem) of stage kl's weight rows and token rows
@@ -687,6 +540,19 @@ __global__ __launch_bounds__(4 * BM / FM, OCC) void gemm_big(const uint8_t* __re
       const uint8_t* base = reinterpret_cast<const uint8_t*>(abase ^ ((wbase ^ abase) & sel));
       const int kl = isw ? klw : kla;
       dma16s(base, doff[i] + static_cast<uint32_t>(kl) * KB, (isw ? wdst : adst) + i * 1024);
+    };
+    // stage 0 when it is the partial one
+    auto dma_tail = [&](uint32_t wdst, uint32_t adst, int i) {
+      const int blk = kW3 ? (i < kW4 ? wave * kW4 + i : BN / 8 + wave * kA4 + (i - kW4)) : wave * kLoads + i;
+      const int row = blk * 8 + lrow;
+      const int kb = (lpos ^ S::f(row)) << 4;
+      const uint8_t* p;
+      if (i < iw) {  // wave-uniform
+        p = W + min(n0 + row, n_last) * ldw + (K - tail + kb);
+      } else {
+        p = A + min(m0 + (row - BN), m_last) * lda + (K - tail + kb);
+      }
+      dma16(kb < tail ? p : kZeroChunk, (i < iw ? wdst : adst) + i * 1024);
     };
     // bases such that DMA i lands at base + i * 1024
     const uint32_t smem_off = lds_offset(smem);
@@ -752,7 +618,9 @@ __global__ __launch_bounds__(4 * BM / FM, OCC) void gemm_big(const uint8_t* __re
 #pragma unroll
         for (int m = 0; m < kLoads; ++m) {
           const int i = dma_at(m);
-          if (i < iw) {
+          if (s == 0 && tail_here) {
+            dma_tail(wd, ad, i);
+          } else if (i < iw) {
             if (s < nk) dma_one(s, 0, wd, ad, i);
           } else if (s < 2 && s < nk) {
             dma_one(0, s, wd, ad, i);
@@ -769,7 +637,10 @@ __global__ __launch_bounds__(4 * BM / FM, OCC) void gemm_big(const uint8_t* __re
         if (s < nk) {
           const uint32_t wd = wdst_of(s), ad = adst_of(s);
 #pragma unroll
-          for (int i = 0; i < kLoads; ++i) dma_one(s, s, wd, ad, i);
+          for (int i = 0; i < kLoads; ++i) {
+            if (s == 0 && tail_here) dma_tail(wd, ad, i);
+            else dma_one(s, s, wd, ad, i);
+          }
         }
       if (nk >= STAGES) wait_vmcnt<(STAGES - 1) * kLoads>();
       else wait_vmcnt<0>();
@@ -846,8 +717,10 @@ __global__ __launch_bounds__(4 * BM / FM, OCC) void gemm_big(const uint8_t* __re
     wait_vmcnt<0>();  // no DMA may still write LDS when the epilogue reuses it
   } else {
 #pragma unroll
-    for (int s = 0; s < STAGES - 1; ++s)
-      if (s < nk) issue(s);
+    for (int s = 0; s < STAGES - 1; ++s) {
+      if (s == 0 && tail_here) issue(s, std::true_type{});
+      else if (s < nk) issue(s, std::false_type{});
+    }
     for (int kt = 0; kt < nk; ++kt) {
       // Loads of stages kt+1 .. kt+STAGES-2 may stay in flight.
       if (kt + STAGES - 2 < nk) wait_vmcnt<(STAGES - 2) * kLoads>();
@@ -855,7 +728,7 @@ __global__ __launch_bounds__(4 * BM / FM, OCC) void gemm_big(const uint8_t* __re
       asm volatile("" ::: "memory");
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
-      if (kt + STAGES - 1 < nk) issue(kt + STAGES - 1);
+      if (kt + STAGES - 1 < nk) issue(kt + STAGES - 1, std::false_type{});
       compute(smem + (kt % STAGES) * kStage);
     }
   }
@@ -1426,70 +1299,6 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny(const uint8_t* __restr
 // Host dispatch
 // ---------------------------------------------------------------------------
 
-template <int BN, int BM, int WGN, int WGM, bool GLU>
-int launch_lds(const uint8_t* a, int64_t lda, const uint8_t* w, int64_t ldw, int64_t K, const Epi& e,
-               hipStream_t st) {
-  const int64_t tiles_m = (e.M + BM - 1) / BM;
-  const int64_t tiles_n = (e.N + BN - 1) / BN;
-  const int64_t grid = tiles_m * tiles_n;
-  if (grid > 0x7FFFFFFFLL) return IFX_ERR_UNSUPPORTED;
-  hipLaunchKernelGGL((gemm_lds<BN, BM, WGN, WGM, GLU>), dim3(static_cast<unsigned>(grid)),
-                     dim3(WGN * WGM * 64), 0, st, a, lda, w, ldw, K, static_cast<int>(tiles_m), e);
-  return launch_status();
-}
-
-// Large-M launch plan: tiles and, when there are too few tiles to fill the
-// GPU, a K split (each slice at least 4 stages) finished by splitk_reduce.
-struct BigPlan {
-  int64_t tiles_m, tiles_n;
-  int ksplit;
-  int64_t kstages;  // K stages per slice
-  size_t ws_bytes;  // fp32 partials of all slices
-};
-
-__host__ inline BigPlan big_plan(int64_t M, int64_t N, int64_t K, int bm, int bn, int kb) {
-  BigPlan p{};
-  p.tiles_m = (M + bm - 1) / bm;
-  p.tiles_n = (N + bn - 1) / bn;
-  const int64_t tiles = p.tiles_m * p.tiles_n;
-  const int64_t nk = K / kb;
-  int64_t s = 1;
-  if (tiles < 192) {
-    // As many slices as keep the grid within one workgroup per CU: a grid of
-    // 1-2 workgroups per CU leaves the CUs that get two the critical path
-    // (measured: 816x2048x16384 51 vs 57 us at 224 vs 336 workgroups;
-    // 1024x2048x11008 44 vs 51 us at 256 vs 320).
-    s = 256 / tiles;
-    if (s > nk / 4) s = nk / 4;
-    if (s < 1) s = 1;
-  }
-  p.kstages = (nk + s - 1) / s;
-  p.ksplit = static_cast<int>((nk + p.kstages - 1) / p.kstages);
-  p.ws_bytes = p.ksplit > 1 ? static_cast<size_t>(p.ksplit) * M * N * sizeof(float) : 0;
-  return p;
-}
-
-template <int BM, int BN, int KB, int STAGES, int OCC, bool GLU, int FM = 2>
-int launch_big(const uint8_t* a, int64_t lda, const uint8_t* w, int64_t ldw, int64_t K, const Epi& e,
-               void* ws, size_t ws_bytes, hipStream_t st) {
-  const BigPlan p = big_plan(e.M, e.N, K, BM, BN, KB);
-  if (p.tiles_m * p.tiles_n * p.ksplit > 0x7FFFFFF0LL) return IFX_ERR_UNSUPPORTED;
-  Partials part{nullptr, e.N, p.kstages};
-  if (p.ksplit > 1) {
-    if (!ws || ws_bytes < p.ws_bytes || !aligned16(ws)) return IFX_ERR_WORKSPACE;
-    part.base = static_cast<float*>(ws);
-  }
-  const TileMap t = make_tile_map(p.tiles_m, p.tiles_n, p.ksplit);
-  hipLaunchKernelGGL((gemm_big<BM, BN, KB, STAGES, OCC, GLU, FM>), dim3(static_cast<unsigned>(8 * t.per_xcd)), dim3(4 * BM / FM),
-                     0, st, a, lda, w, ldw, K, t, e, part);
-  if (p.ksplit > 1) {
-    const int64_t threads = e.M * ((GLU ? e.N / 2 : e.N) / 4);
-    hipLaunchKernelGGL((splitk_reduce<GLU>), dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, st,
-                       part, p.ksplit, e);
-  }
-  return launch_status();
-}
-
 template <int MB, int NBW, int WAVES>
 void launch_skinny_w(const SkinnyPlan& p, const uint8_t* a, int64_t lda, const uint8_t* w, int64_t ldw, int64_t K,
                      const Epi& e, const SkArgs& sp, hipStream_t st) {
@@ -1563,66 +1372,125 @@ __global__ __launch_bounds__(256) void pack_skinny_kernel(const uint8_t* __restr
   *reinterpret_cast<v4i*>(out + c * 16) = v;
 }
 
-// Large-M configurations (all with 128-byte K stages, so K % 128 == 0): see
-// pick_big below.
-constexpr int kBigKB = 128;
-
-// Every M past the skinny range (M > 64) with K % 128 == 0 takes gemm_big; its
-// small-grid configurations beat gemm_lds there by 3-5x (65x2048x2048 8.8 vs
-// 33 us, 128x4096x8192 22.5 vs 97 us), so gemm_lds only serves K % 128 != 0.
-inline bool big_path(int64_t M, int64_t K) { return M > kSkinnyMaxM && K % kBigKB == 0; }
-
-// Large-M configuration for a shape:
+// Large-M configurations, all with 128-byte K stages:
 //  * kWide / kWide192: 256 tokens x 256 (or 192) weight rows per workgroup, one
-//    workgroup per CU. 256 x 256 tiles run the 4-wave register-pipelined form
-//    (C5 up 8192x14336x3072 GELU 341 -> 317 us, C5 qkv 247 -> 224 us, C3 gate|up
-//    73 -> 69 us against 8 waves of 128 x 64), or 8 waves when an operand
-//    spans 4 GiB or more (32-bit DMA offsets); 256 x 192 tiles likewise. 192-row tiles are taken when they need
-//    fewer tile rounds on the 256 CUs, weighted by tile height and efficiency:
-//    e.g. an 8192 x 3072 output is 384 tiles of 256 rows (a half-empty second
-//    round) but 512 tiles of 192 rows (two full rounds): 329 -> 302 us for
-//    K = 14336; a GLU output of 1024 x 22016 is 344 tiles of 256 but 460 of 192.
-//  * kSmall: fewer than 192 tiles of 256 x 256 and K <= 4096 -- 64 tokens x
-//    128 weight rows, 128-byte stages, 4 waves of 64 x 32 (short MFMA chains
+//    workgroup per CU, the 4-wave register-pipelined form (C5 up 8192x14336x3072
+//    GELU 341 -> 317 us, C5 qkv 247 -> 224 us, C3 gate|up 73 -> 69 us against 8
+//    waves of 128 x 64), or 8 waves when an operand spans 4 GiB or more (32-bit
+//    DMA offsets);
+//  * kNarrow / kNarrow192: 128 tokens x 256 (or 192) weight rows, the
+//    register-pipelined 4 waves of 64 x 128 (64 x 96) with a 3-stage ring (8 waves
+//    of 128 x 32 and two stages for operands past 4 GiB);
+//  * kSmall: 64 tokens x 128 weight rows, 4 waves of 64 x 32 (short MFMA chains
 //    per wave: the loop is latency-bound at these sizes), a 3-stage ring, two
-//    workgroups per CU, usually no split (1024 x 2560 x 2048: 28 us with split-K
-//    narrow tiles, 15.7 us with 2 waves of 64 x 64 and 64-byte stages, 12.1 us
-//    with a 2-stage ring; weights streamed from HBM with bias and residual,
-//    2 -> 3 stages: 1024 x 2560 18.2 -> 15.5 us, 1024 x 2048 15.5 -> 12.3 us);
-//  * kSmall32: as kSmall with 32-token tiles (2 waves of 64 x 32) when 64-token
-//    tiles would give fewer than 256 workgroups (200 x 2560 x 2048 10.7 -> 8.8 us,
-//    512 x 1024 x 2048 12.4 -> 10.6 us; at 256 or more the 64-token tiles win:
-//    1024 x 2560 x 2048 12.2 against 15.2 us). A 4-stage ring when the grid fits
-//    one workgroup per CU, else 3 stages and two per CU (streamed weights: 200 x
-//    2560 x 2048 16.2 -> 10.5 us, 300 x 3072 x 3072 23.0 -> 14.4 us, 816 x 2048 x
-//    2048 16.7 -> 14.0 us against 2 stages);
-//  * kNarrow: fewer than 192 tiles and a longer K -- 128 tokens x 256 weight
-//    rows, the register-pipelined 4 waves of 64 x 128 with a 3-stage ring
-//    (144 KB) when the 32-bit DMA offsets fit (else 8 waves of 128 x 32, two
-//    stages), 128-byte stages, plus split K. 816 x 2048 x 16384: 44.1 us with 8
-//    waves, 42.8 pipelined with two stages, 41.0 with three; with the weights
-//    streamed from HBM 52.0 -> 42.4 us (two -> three stages), 1024 x 2048 x 11008
-//    44.2 -> 39.3 us. (44 us with 4 waves of 128 x 64 and 64-byte stages; the
-//    64 x 128 / 32 x 128 tiles without a split, re-measured on the current
-//    kernels: 1024 x 2048 x 11008 44.3 against 40.2 us, 816 x 2048 x 16384 56-60
-//    against 43-45 us.)
-enum class BigCfg { kWide, kWide192, kSmall, kSmall32, kNarrow };
+//    workgroups per CU;
+//  * kSmall32: as kSmall with 32-token tiles (2 waves of 64 x 32).
+// Narrow and small tiles stream more operand bytes L2 -> LDS per FLOP (which is
+// what bounds every one of them), wide ones quantize the output into fewer
+// workgroups, and a K split writes and re-reads fp32 partials.
+enum class BigCfg { kWide, kWide192, kNarrow, kNarrow192, kSmall, kSmall32 };
 
-inline BigCfg pick_big(int64_t M, int64_t N, int64_t K, bool glu) {
-  const int64_t tm = (M + 255) / 256;
-  const int64_t t256 = tm * ((N + 255) / 256);
-  if (t256 < 192) {
-    if (K > 4096) return BigCfg::kNarrow;
-    return ((M + 63) / 64) * ((N + 127) / 128) < 256 ? BigCfg::kSmall32 : BigCfg::kSmall;
+// What a launch of workgroups of `st` K stages each takes, in us: `slots`
+// workgroups are resident at once, every full round before the last one takes
+// round + st * t(slots), the last one of n workgroups fixed + st * t(n), with
+//   t(n) = stage + load * min(n, 256) / 256 (+ pair when some CU has two)
+// and `ragged` times more per stage when rows do not start on 128-byte lines
+// (K % 128 != 0: every 128-byte piece of a row then spans two). The constants are
+// a least-squares fit to 4100 launches measured on MI355X (210 shapes of 65-8192
+// tokens, 500-32768 weight rows and K 512-16384, each with every configuration
+// and several splits; 8% rms). Choosing by the fit takes 1.2% longer than the
+// best measured choice over those shapes (geometric mean); the thresholds it
+// replaced (256-token tiles from 192 of them on, else split 128 x 256 tiles for
+// K > 4096, else 64 x 128 or 32 x 128) took 14% longer, e.g. 6000x1152x4304 60.5
+// -> 39.3 us, 1155x5568x12320 GeGLU 164 -> 106, 1500x3072x3072 28.3 -> 21.1,
+// 333x22016x2048 33.7 -> 24.3; the worst shape against them loses 5% (K % 128 == 0).
+struct BigCost {
+  int bm, bn, slots;
+  double fixed, round, stage, load, pair, ragged;
+};
+constexpr BigCost kBigCost[] = {
+    {256, 256, 256, 10.6, 7.1, 0.880, 0.096, 0.0, 0.25},    // kWide
+    {256, 192, 256, 9.9, 6.4, 0.671, 0.174, 0.0, 0.25},     // kWide192
+    {128, 256, 256, 8.0, 5.4, 0.537, 0.160, 0.0, 0.39},     // kNarrow
+    {128, 192, 256, 7.5, 5.0, 0.417, 0.146, 0.0, 0.42},     // kNarrow192
+    {64, 128, 512, 4.6, 1.9, 0.289, 0.074, 0.246, 0.25},    // kSmall
+    {32, 128, 512, 4.4, 2.5, 0.246, 0.037, 0.164, 0.35},    // kSmall32
+};
+// a K split: the reduce launch, and writing and reading the partials
+constexpr double kSplitFixed = 2.9, kSplitPerByte = 0.27e-6;
+
+inline double big_cost(const BigCost& c, int64_t workgroups, int64_t st, bool ragged) {
+  const int64_t rounds = (workgroups - 1) / c.slots, last = workgroups - rounds * c.slots;
+  auto t = [&](int64_t n) {
+    return (c.stage + c.load * static_cast<double>(std::min<int64_t>(n, 256)) / 256 + (n > 256 ? c.pair : 0.0)) *
+           (ragged ? 1.0 + c.ragged : 1.0);
+  };
+  return rounds * (c.round + st * t(c.slots)) + c.fixed + st * t(last);
+}
+
+// Most K slices of a shape: only outputs of few tiles are split, each slice at
+// least 4 stages deep. This bounds the workspace; the plan may take fewer.
+inline int64_t max_split(int64_t M, int64_t N, int64_t nk) {
+  const int64_t tiles = nk > 32 ? ((M + 127) / 128) * ((N + 255) / 256) : ((M + 31) / 32) * ((N + 127) / 128);
+  const int64_t s = tiles < 192 ? std::max<int64_t>(1, std::min(256 / tiles, nk / 4)) : 1;
+  const int64_t kst = (nk + s - 1) / s;
+  return (nk + kst - 1) / kst;  // no empty slice
+}
+
+struct BigPlan {
+  BigCfg cfg;
+  int ksplit;
+  int64_t kstages;  // K stages per slice
+};
+
+inline BigPlan big_plan(int64_t M, int64_t N, int64_t K, bool may_split) {
+  const int64_t nk = (K + kBK - 1) / kBK;
+  const int64_t most = may_split ? max_split(M, N, nk) : 1;
+  BigPlan best{};
+  double best_t = 0;
+  for (int i = 0; i < static_cast<int>(std::size(kBigCost)); ++i) {
+    const BigCost& c = kBigCost[i];
+    const int64_t tiles = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
+    for (int64_t s = 1; s <= most && (s == 1 || tiles * s <= 512); ++s) {
+      const int64_t kst = (nk + s - 1) / s, ks = (nk + kst - 1) / kst;
+      const double t = big_cost(c, tiles * ks, kst, K % kBK != 0) +
+                       (ks > 1 ? kSplitFixed + kSplitPerByte * static_cast<double>(4 * ks * M * N) : 0.0);
+      if (best_t == 0 || t < best_t) {
+        best_t = t;
+        best = {static_cast<BigCfg>(i), static_cast<int>(ks), kst};
+      }
+    }
   }
-  (void)glu;  // GLU tiles take the same shapes (16-row gate|up blocks divide 192)
-  {
-    const int64_t t192 = tm * ((N + 191) / 192);
-    // a 192-row tile does ~15% less work per unit time than a 256-row one
-    // (measured: 8192x9216x3072, 6 full rounds of 192 vs 4.5 of 256, is 2.5% slower)
-    if (((t192 + 255) / 256) * 192 * 115 < ((t256 + 255) / 256) * 256 * 100) return BigCfg::kWide192;
+  return best;
+}
+
+// Workspace of a shape: the fp32 partials of the most slices it may be cut into.
+inline size_t split_bytes(int64_t M, int64_t N, int64_t K) {
+  const int64_t s = max_split(M, N, (K + kBK - 1) / kBK);
+  return s > 1 ? static_cast<size_t>(s) * M * N * sizeof(float) : 0;
+}
+
+// Whether a call may run without the workspace its K split wants: a K that is
+// no multiple of 128 needed none before such shapes were split, so a caller
+// without it (a stream being captured, a fixed scratch buffer) is still served,
+// by unsplit tiles.
+inline bool split_optional(int64_t K) { return K % kBK != 0; }
+
+template <int BM, int BN, int KB, int STAGES, int OCC, bool GLU, int FM = 2>
+int launch_big(const uint8_t* a, int64_t lda, const uint8_t* w, int64_t ldw, int64_t K, const Epi& e,
+               void* ws, const BigPlan& p, hipStream_t st) {
+  const int64_t tiles_m = (e.M + BM - 1) / BM, tiles_n = (e.N + BN - 1) / BN;
+  if (tiles_m * tiles_n * p.ksplit > 0x7FFFFFF0LL) return IFX_ERR_UNSUPPORTED;
+  const Partials part{p.ksplit > 1 ? static_cast<float*>(ws) : nullptr, e.N, p.kstages};
+  const TileMap t = make_tile_map(tiles_m, tiles_n, p.ksplit);
+  hipLaunchKernelGGL((gemm_big<BM, BN, KB, STAGES, OCC, GLU, FM>), dim3(static_cast<unsigned>(8 * t.per_xcd)), dim3(4 * BM / FM),
+                     0, st, a, lda, w, ldw, K, t, e, part);
+  if (p.ksplit > 1) {
+    const int64_t threads = e.M * ((GLU ? e.N / 2 : e.N) / 4);
+    hipLaunchKernelGGL((splitk_reduce<GLU>), dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, st,
+                       part, p.ksplit, e);
   }
-  return BigCfg::kWide;
+  return launch_status();
 }
 
 // The 4-wave kernel forms DMA addresses as a 32-bit byte offset (row * ld, a
@@ -1636,30 +1504,27 @@ inline bool dma32_ok(int64_t M, int64_t N, int64_t lda, int64_t ldw) {
 template <bool GLU>
 int launch_large(const uint8_t* a, int64_t lda, const uint8_t* w, int64_t ldw, int64_t K, const Epi& e, void* ws,
                  size_t ws_bytes, hipStream_t st) {
-  switch (pick_big(e.M, e.N, K, GLU)) {
+  const size_t need = split_bytes(e.M, e.N, K);
+  const bool have = need == 0 || (ws && ws_bytes >= need && aligned16(ws));
+  if (!have && !split_optional(K)) return IFX_ERR_WORKSPACE;
+  const BigPlan p = big_plan(e.M, e.N, K, have);
+  const bool dma32 = dma32_ok(e.M, e.N, lda, ldw);
+  switch (p.cfg) {
     case BigCfg::kWide192:
-      if (dma32_ok(e.M, e.N, lda, ldw))
-        return launch_big<256, 192, 128, 2, 1, GLU, 4>(a, lda, w, ldw, K, e, ws, ws_bytes, st);
-      if constexpr (!GLU) return launch_big<256, 192, 128, 2, 1, GLU>(a, lda, w, ldw, K, e, ws, ws_bytes, st);
-      [[fallthrough]];  // operands past 4 GiB with GLU: 8 waves of 256 x 256 (no split at this size)
+      if (dma32) return launch_big<256, 192, 128, 2, 1, GLU, 4>(a, lda, w, ldw, K, e, ws, p, st);
+      if constexpr (!GLU) return launch_big<256, 192, 128, 2, 1, GLU>(a, lda, w, ldw, K, e, ws, p, st);
+      [[fallthrough]];  // operands past 4 GiB with GLU: 8 waves of 256 x 256
     case BigCfg::kWide:
-      if (dma32_ok(e.M, e.N, lda, ldw))
-        return launch_big<256, 256, 128, 2, 1, GLU, 4>(a, lda, w, ldw, K, e, ws, ws_bytes, st);
-      return launch_big<256, 256, 128, 2, 1, GLU>(a, lda, w, ldw, K, e, ws, ws_bytes, st);
-    case BigCfg::kSmall:
-      return launch_big<64, 128, 128, 3, 2, GLU, 1>(a, lda, w, ldw, K, e, ws, ws_bytes, st);
-    case BigCfg::kSmall32: {
-      // a grid that fits one workgroup per CU takes a 4-stage ring (80 KB);
-      // larger grids 3 stages, two workgroups per CU
-      const BigPlan p = big_plan(e.M, e.N, K, 32, 128, 128);
-      if (p.tiles_m * p.tiles_n * p.ksplit <= 256)
-        return launch_big<32, 128, 128, 4, 1, GLU, 1>(a, lda, w, ldw, K, e, ws, ws_bytes, st);
-      return launch_big<32, 128, 128, 3, 2, GLU, 1>(a, lda, w, ldw, K, e, ws, ws_bytes, st);
-    }
+      if (dma32) return launch_big<256, 256, 128, 2, 1, GLU, 4>(a, lda, w, ldw, K, e, ws, p, st);
+      return launch_big<256, 256, 128, 2, 1, GLU>(a, lda, w, ldw, K, e, ws, p, st);
+    case BigCfg::kSmall: return launch_big<64, 128, 128, 3, 2, GLU, 1>(a, lda, w, ldw, K, e, ws, p, st);
+    case BigCfg::kSmall32: return launch_big<32, 128, 128, 3, 2, GLU, 1>(a, lda, w, ldw, K, e, ws, p, st);
+    case BigCfg::kNarrow192:
+      if (dma32) return launch_big<128, 192, 128, 3, 1, GLU, 2>(a, lda, w, ldw, K, e, ws, p, st);
+      [[fallthrough]];
     default:
-      if (dma32_ok(e.M, e.N, lda, ldw))
-        return launch_big<128, 256, 128, 3, 1, GLU, 2>(a, lda, w, ldw, K, e, ws, ws_bytes, st);
-      return launch_big<128, 256, 128, 2, 1, GLU, 1>(a, lda, w, ldw, K, e, ws, ws_bytes, st);
+      if (dma32) return launch_big<128, 256, 128, 3, 1, GLU, 2>(a, lda, w, ldw, K, e, ws, p, st);
+      return launch_big<128, 256, 128, 2, 1, GLU, 1>(a, lda, w, ldw, K, e, ws, p, st);
   }
 }
 
@@ -1671,16 +1536,10 @@ using namespace ifx;
 extern "C" {
 
 size_t ifx_fp8_linear_workspace_size(int64_t M, int64_t N, int64_t K, int epilogue) {
+  (void)epilogue;  // every epilogue of a shape takes the same slices
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   if (M <= kSkinnyMaxM) return 0;  // the skinny kernel needs no workspace
-  if (!big_path(M, K)) return 0;
-  switch (pick_big(M, N, K, (epilogue & (IFX_EPI_GEGLU | IFX_EPI_SWIGLU)) != 0)) {
-    case BigCfg::kWide192: return big_plan(M, N, K, 256, 192, 128).ws_bytes;
-    case BigCfg::kWide: return big_plan(M, N, K, 256, 256, 128).ws_bytes;
-    case BigCfg::kSmall: return big_plan(M, N, K, 64, 128, 128).ws_bytes;
-    case BigCfg::kSmall32: return big_plan(M, N, K, 32, 128, 128).ws_bytes;
-    default: return big_plan(M, N, K, 128, 256, 128).ws_bytes;
-  }
+  return split_bytes(M, N, K);
 }
 
 }  // extern "C"
@@ -1735,9 +1594,9 @@ struct QlWorkspace {
   size_t gemm, q, scale, partial, total;
 };
 
-QlWorkspace ql_workspace(int64_t M, int64_t N, int64_t K, int epilogue, int scale_mode) {
+QlWorkspace ql_workspace(int64_t M, int64_t N, int64_t K, int epilogue, int scale_mode, bool may_split = true) {
   QlWorkspace w{};
-  w.gemm = round256(ifx_fp8_linear_workspace_size(M, N, K, epilogue));
+  w.gemm = may_split ? round256(ifx_fp8_linear_workspace_size(M, N, K, epilogue)) : 0;
   w.q = round256(static_cast<size_t>(M) * K);
   w.scale = round256(static_cast<size_t>(M) * sizeof(float));
   w.partial = scale_mode == IFX_SCALE_TENSOR ? round256(ifx_quant_tensor_workspace_size(M * K)) : 0;
@@ -1771,19 +1630,10 @@ int ifx_fp8_linear(const void* a, int64_t lda, const float* sa, const void* w, i
     const SkinnyPlan p = skinny_plan(M, N, K, glu);
     return glu ? launch_skinny<2>(p, A, lda, Wt, ldw, K, e, st) : launch_skinny<1>(p, A, lda, Wt, ldw, K, e, st);
   }
-  if (big_path(M, K)) {
-    const int64_t out_bytes = M * (glu ? N / 2 : N) * static_cast<int64_t>(sizeof(uint16_t));
-    e.nt_out = out_bytes >= kNtOutBytes;
-    return glu ? launch_large<true>(A, lda, Wt, ldw, K, e, workspace, ws_bytes, st)
-               : launch_large<false>(A, lda, Wt, ldw, K, e, workspace, ws_bytes, st);
-  }
-  // Grids under one round of 256 x 128 tiles take 64 x 64 tiles (4 waves of
-  // 32 x 32): 100x2560x2064 35.5 -> 10.5 us, 1000x2048x2064 39.5 -> 16.8 us.
-  if (((M + 127) / 128) * ((N + 255) / 256) < 256)
-    return glu ? launch_lds<64, 64, 2, 2, true>(A, lda, Wt, ldw, K, e, st)
-               : launch_lds<64, 64, 2, 2, false>(A, lda, Wt, ldw, K, e, st);
-  return glu ? launch_lds<256, 128, 2, 2, true>(A, lda, Wt, ldw, K, e, st)
-             : launch_lds<256, 128, 2, 2, false>(A, lda, Wt, ldw, K, e, st);
+  const int64_t out_bytes = M * (glu ? N / 2 : N) * static_cast<int64_t>(sizeof(uint16_t));
+  e.nt_out = out_bytes >= kNtOutBytes;
+  return glu ? launch_large<true>(A, lda, Wt, ldw, K, e, workspace, ws_bytes, st)
+             : launch_large<false>(A, lda, Wt, ldw, K, e, workspace, ws_bytes, st);
 }
 
 int ifx_fp8_linear_qkv_rope(const void* a, int64_t lda, const float* sa, const void* w, int64_t ldw,
@@ -1876,7 +1726,8 @@ int ifx_quant_linear(const void* x, int64_t ldx, int scale_mode, const void* w, 
                                     M, N, K);
   if (rc != IFX_OK || M == 0) return rc;
   // the stand-alone quantizer into the workspace, then the GEMM
-  const QlWorkspace ql = ql_workspace(M, N, K, epilogue, scale_mode);
+  QlWorkspace ql = ql_workspace(M, N, K, epilogue, scale_mode);
+  if (ws_bytes < ql.total && split_optional(K)) ql = ql_workspace(M, N, K, epilogue, scale_mode, false);
   if (!workspace || ws_bytes < ql.total || (reinterpret_cast<uintptr_t>(workspace) & 255u)) return IFX_ERR_WORKSPACE;
   uint8_t* base = static_cast<uint8_t*>(workspace);
   void* gws = base;
@@ -1958,7 +1809,7 @@ int ifx_quant_linear_noalloc(const void* x, int64_t ldx, int scale_mode, const v
   // every contract check before the scratch is touched: a rejected call launches nothing
   int rc = check_quant_linear(x, ldx, scale_mode, w, ldw, sw, bias, residual, ldr, gate, epilogue, out, ldo, M, N, K);
   if (rc != IFX_OK || M == 0) return rc;
-  const size_t need = ql_workspace(M, N, K, epilogue, scale_mode).total;
+  const size_t need = ql_workspace(M, N, K, epilogue, scale_mode, !split_optional(K)).total;
   if (need > kScratchBytes) return IFX_ERR_SCRATCH;
   void* ws = scratch_ptr(&rc);
   if (!ws) return rc;

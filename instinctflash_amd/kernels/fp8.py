@@ -135,28 +135,32 @@ _WORKSPACES: dict = {}
 _RETIRED: list = []
 
 
-def _workspace(nbytes: int, device, stream: int):
-    """Workspace per (device, stream), reused by every call on that stream
+def _workspace(nbytes: int, device, stream: int, least: int | None = None):
+    """(buffer, usable bytes) of the workspace per (device, stream), reused by every call on that stream
     (calls on one stream are ordered). It holds split-K partial sums, which
     every call writes before it reads them, so it needs no initialisation.
 
     A buffer outgrown by a later call is kept alive (never freed), because a
     captured HIP graph may still hold its address. Growing while the stream is
     being captured raises instead: run the captured calls once eagerly first,
-    so the buffer is already large enough."""
+    so the buffer is already large enough. A call that can also run with
+    ``least`` bytes (without its K split) takes what there is under capture."""
     if nbytes == 0:
-        return None
+        return None, 0
     key = (device.index, stream)
     ws = _WORKSPACES.get(key)
     if ws is None or ws.numel() < nbytes:
         if torch.cuda.is_current_stream_capturing():
+            have = 0 if ws is None else ws.numel()
+            if least is not None and have >= least:
+                return ws, have
             raise RuntimeError(f"the FP8 workspace of this stream must grow to {nbytes} bytes during HIP graph "
                                "capture; run the captured calls once before capturing")
         if ws is not None:
             _RETIRED.append(ws)
         ws = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
         _WORKSPACES[key] = ws
-    return ws
+    return ws, nbytes
 
 
 # ---------------------------------------------------------------------------
@@ -354,7 +358,7 @@ def _linear(a, sa, w: Fp8Weight, out, flags, residual=None, gate=None, use_scale
     lib = _lib.load()
     stream = _stream(a.device)
     nbytes = lib.ifx_fp8_linear_workspace_size(M, N, K, flags)
-    ws = _workspace(nbytes, a.device, stream)
+    ws, nbytes = _workspace(nbytes, a.device, stream, 0 if K % 128 else None)
     _lib.check(lib.ifx_fp8_linear(_ptr(a_t), lda, _ptr(sa) if use_scales else None, _ptr(w.w), ldw,
                                   _ptr(sw), _ptr(bias), _ptr(residual), ldr, _ptr(gate), flags,
                                   _ptr(out), ldo, M, N, K, _ptr(ws), nbytes, stream), "ifx_fp8_linear")
@@ -424,7 +428,8 @@ def quant_linear(x: torch.Tensor, w: Fp8Weight, out: torch.Tensor | None = None,
     lib = _lib.load()
     stream = _stream(x.device)
     nbytes = lib.ifx_quant_linear_workspace_size(M, N, K, flags, mode)
-    ws = _workspace(nbytes, x.device, stream)
+    least = nbytes - -(-lib.ifx_fp8_linear_workspace_size(M, N, K, flags) // 256) * 256 if K % 128 else None
+    ws, nbytes = _workspace(nbytes, x.device, stream, least)
     _lib.check(lib.ifx_quant_linear(_ptr(x), ldx, mode, _ptr(w.w), ldw, _ptr(sw), _ptr(bias), _ptr(residual), ldr,
                                     _ptr(gate), flags, _ptr(out), ldo, M, N, K, _ptr(a_scale), _ptr(ws), nbytes,
                                     stream), "ifx_quant_linear")

@@ -189,7 +189,7 @@ def linear_qkv_rope(a, a_scale, w, q_out, k_out, v_out, *, inv_freq=None, pos=No
     lib = _lib.load()
     stream = _stream(dev)
     nbytes = lib.ifx_fp8_linear_workspace_size(M, N, K, 0)
-    ws = _workspace(nbytes, dev, stream)
+    ws, nbytes = _workspace(nbytes, dev, stream)
     _lib.check(lib.ifx_fp8_linear_qkv_rope(
         _ptr(a_t), lda, _ptr(a_scale), _ptr(w.w), ldw, _ptr(w.scale), _ptr(w.bias), flags,
         _ptr(pos) if inv_freq is not None else None, ldpos, _ptr(inv_freq), HQ, HKV, HD,

@@ -210,6 +210,59 @@ def test_unaligned_k_lds_path(gpu, oracle_mod, M, N, K, act):
            residual=res)
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (70, 256, 16), (65, 512, 112),         # K shorter than one stage (32 x 128 tiles)
+    (100, 768, 144), (900, 4096, 272),     # 32- and 64-token tiles
+    (100, 512, 4112), (768, 1152, 4304),   # split K: the partial stage is the first slice's
+    (2000, 3008, 272),                     # 128 x 192 tiles
+    (3000, 4096, 1136), (8192, 3072, 208)])  # 256 x 256 and 256 x 192 tiles
+def test_k_tail_stage(gpu, oracle_mod, M, N, K):
+    # K % 128 != 0: the partial stage must multiply zeros past K, whatever lies
+    # there. Both operands are row-strided with NaN codes right after K.
+    from instinctflash_amd.kernels import Fp8Weight
+    qa, sa, fw, g = _make(gpu, M, N, K, seed=M + K, bias=True)
+    ap = torch.full((M, K + 128), 0x7F, dtype=torch.uint8, device=gpu)
+    wp = torch.full((N, K + 128), 0x7F, dtype=torch.uint8, device=gpu)
+    ap[:, :K] = qa.view(torch.uint8)
+    wp[:, :K] = fw.w.view(torch.uint8)
+    w = Fp8Weight(wp.view(torch.float8_e4m3fn)[:, :K], fw.scale, fw.bias)
+    res = torch.randn((M, N), generator=g).to(torch.bfloat16)
+    _check(gpu, oracle_mod, ap.view(torch.float8_e4m3fn)[:, :K], sa, w, f"tail {M}x{N}x{K}", ref_w=fw, residual=res)
+
+
+@pytest.mark.parametrize("M,N,K,act,gate", [(1500, 3072, 512, "gelu_tanh", False), (2000, 3008, 384, None, True),
+                                            (1100, 4000, 400, "geglu", False), (816, 2048, 16384, "swiglu", False)])
+def test_128x192_tiles(gpu, oracle_mod, M, N, K, act, gate):
+    # 128 tokens x 192 weight rows (the last with split K): token and weight tiles end ragged, GLU pairs
+    # of 192 = 6 x 32 packed rows, gated residual
+    from instinctflash_amd.kernels import pack_glu
+    qa, sa, fw, g = _make(gpu, M, N, K, seed=M, bias=True)
+    glu = act in ("geglu", "swiglu")
+    n_out = N // 2 if glu else N
+    res = torch.randn((M, n_out), generator=g).to(torch.bfloat16)
+    _check(gpu, oracle_mod, qa, sa, pack_glu(fw) if glu else fw, f"narrow192 {M}x{N}x{K}", ref_w=fw, act=act,
+           residual=res, gate=torch.rand(n_out, generator=g).to(torch.bfloat16) if gate else None)
+
+
+def test_k_tail_without_workspace(gpu, oracle_mod):
+    # K % 128 != 0 needs no workspace: captured on a stream that has none, the call runs without its K split
+    from instinctflash_amd.kernels import linear
+    M, N, K = 300, 1152, 4304
+    qa, sa, fw, _ = _make(gpu, M, N, K, seed=11, bias=True)
+    out = torch.empty((M, N), device=gpu)
+    linear(qa, sa, fw, out=out)
+    split = out.clone()
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.graph(graph, stream=side):
+        linear(qa, sa, fw, out=out)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        _assert_close(_f(out), _ref(oracle_mod, qa, sa, fw), "no workspace")
+    assert torch.allclose(out, split, rtol=0, atol=1e-4 * split.abs().max().item())
+
+
 @pytest.mark.parametrize("M,N,K,act", [(65, 2048, 2048, None), (100, 2560, 2048, "gelu_tanh"), (128, 1024, 4096, None),
                                        (96, 1056, 8192, None), (96, 4096, 1024, "geglu"), (72, 2048, 6144, "swiglu")])
 def test_mid_m_large_kernel(gpu, oracle_mod, M, N, K, act):
