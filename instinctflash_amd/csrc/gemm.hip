@@ -86,9 +86,11 @@ __device__ __forceinline__ float epi_sa(const Epi& e, int64_t m) {
 }
 
 // Weight scales sw[n..n+3] (one shared value with IFX_EPI_SCALAR_SW; 1 if absent).
+// The shared value comes by a scalar load: its copy into four registers would
+// otherwise wait for every vector load and DMA issued before it.
 __device__ __forceinline__ float4 epi_sw4(const Epi& e, int64_t n) {
   if (e.sw && (e.flags & IFX_EPI_SCALAR_SW)) {
-    const float v = e.sw[0];
+    const float v = *(const __attribute__((address_space(4))) float*)(reinterpret_cast<uintptr_t>(e.sw));
     return make_float4(v, v, v, v);
   }
   return load_f4_or(e.sw, n, 1.0f);
@@ -380,15 +382,21 @@ __global__ __launch_bounds__(4 * BM / FM, OCC) void gemm_big(const uint8_t* __re
   const int64_t m0 = static_cast<int64_t>(tm) * BM;
   // this workgroup's K stages: [kt0, kt0 + nk); with a partial stage (number
   // 0, `tail` bytes) stage t >= 1 starts at byte t * KB - kshift
-  const int kt0 = static_cast<int>(split * part.kstages);
-  const int nk = static_cast<int>(min((K + KB - 1) / KB - kt0, part.kstages));
-  const int tail = static_cast<int>(K % KB);
+  const int kst = static_cast<int>(part.kstages);
+  const int kt0 = split * kst;
+  const int nk = min(static_cast<int>((static_cast<uint64_t>(K) + KB - 1) / KB) - kt0, kst);
+  const int tail = static_cast<int>(K & (KB - 1));
   const int kshift = tail ? KB : 0;
   const bool tail_here = tail && kt0 == 0;
 
   // Epilogue operands of this lane (column scales, bias, adaLN gate) and this
   // thread's token scale, loaded before the K loop so their latency hides
-  // under it (after the loop they were a serialized round trip per tile).
+  // under it (after the loop they were a serialized round trip per tile). The
+  // 4-wave loops load them after the first stage's DMA: they are about 200
+  // instructions of addresses and flag branches (816x32768x2048 GeGLU and its
+  // 816x2048x16384 down projection 245 -> 243 us for two such layers). The small
+  // tiles load them first: their first barrier would wait for them instead
+  // (1024x2048x2048 11.6 -> 11.8 us).
   constexpr int kCols = GLU ? 16 * kFN : 32 * kFN;  // output columns of a wave tile
   constexpr int kLanesPerRow = kCols / 4;
   // whole rows per 64-lane pass, a power of two (12 lanes per row for 192-row
@@ -404,14 +412,18 @@ __global__ __launch_bounds__(4 * BM / FM, OCC) void gemm_big(const uint8_t* __re
   // lanes past kRowsPerPass whole rows (96-column tiles) have no column of their own
   const bool col_ok = lane < kRowsPerPass * kLanesPerRow && c_out < (GLU ? e.N / 2 : e.N);
   const int64_t np = col_ok ? nw + pc : 0;         // packed weight row (any valid row if unused)
-  const float* bp = (e.flags & IFX_EPI_BIAS) ? e.bias : nullptr;
-  const float4 sw0 = epi_sw4(e, np);
-  const float4 b0 = load_f4_or(bp, np, 0.0f);
-  const float4 sw1 = GLU ? epi_sw4(e, np + 16) : sw0;
-  const float4 b1 = GLU ? load_f4_or(bp, np + 16, 0.0f) : b0;
+  float4 sw0, b0, sw1, b1;
   uint2 g2 = make_uint2(0x3F803F80u, 0x3F803F80u);  // bf16 1.0 x 4
-  if ((e.flags & IFX_EPI_GATE) && col_ok) g2 = *reinterpret_cast<const uint2*>(e.gate + c_out);
-  const float sa_pre = tid < BM ? epi_sa(e, min(m0 + tid, e.M - 1)) : 0.0f;
+  float sa_pre = 0.0f;
+  auto load_epi = [&]() __attribute__((always_inline)) {
+    const float* bp = (e.flags & IFX_EPI_BIAS) ? e.bias : nullptr;
+    sw0 = epi_sw4(e, np);
+    b0 = load_f4_or(bp, np, 0.0f);
+    sw1 = GLU ? epi_sw4(e, np + 16) : sw0;
+    b1 = GLU ? load_f4_or(bp, np + 16, 0.0f) : b0;
+    if ((e.flags & IFX_EPI_GATE) && col_ok) g2 = *reinterpret_cast<const uint2*>(e.gate + c_out);
+    if (tid < BM) sa_pre = epi_sa(e, min(m0 + tid, e.M - 1));
+  };
 
   // DMA load i of a stage covers rows kRowsPerDma*blk .. +kRowsPerDma-1
   // (blk = wave*kLoads + i; weight rows first, then token rows). Rows past N/M
@@ -615,17 +627,18 @@ __global__ __launch_bounds__(4 * BM / FM, OCC) void gemm_big(const uint8_t* __re
 #pragma unroll
       for (int s = 0; s < 3; ++s) {
         const uint32_t wd = wdst_of(s), ad = adst_of(s);
+        if (s == 0 && tail_here) {
 #pragma unroll
-        for (int m = 0; m < kLoads; ++m) {
-          const int i = dma_at(m);
-          if (s == 0 && tail_here) {
-            dma_tail(wd, ad, i);
-          } else if (i < iw) {
-            if (s < nk) dma_one(s, 0, wd, ad, i);
-          } else if (s < 2 && s < nk) {
-            dma_one(0, s, wd, ad, i);
+          for (int m = 0; m < kLoads; ++m) dma_tail(wd, ad, dma_at(m));
+        } else if (s < nk) {
+#pragma unroll
+          for (int m = 0; m < kLoads; ++m) {
+            const int i = dma_at(m);
+            if (i < iw) dma_one(s, 0, wd, ad, i);
+            else if (s < 2) dma_one(0, s, wd, ad, i);
           }
         }
+        if (s == 0) load_epi();
       }
       if (nk >= 3) wait_vmcnt<kLoads + kW4>();  // this wave's A1 W1 W2 may stay in flight
       else if (nk == 2) wait_vmcnt<kLoads>();
@@ -633,15 +646,17 @@ __global__ __launch_bounds__(4 * BM / FM, OCC) void gemm_big(const uint8_t* __re
     } else {
       // prologue: stages 0 .. STAGES-1 in flight, stage 0 landed
 #pragma unroll
-      for (int s = 0; s < STAGES; ++s)
-        if (s < nk) {
-          const uint32_t wd = wdst_of(s), ad = adst_of(s);
+      for (int s = 0; s < STAGES; ++s) {
+        const uint32_t wd = wdst_of(s), ad = adst_of(s);
+        if (s == 0 && tail_here) {
 #pragma unroll
-          for (int i = 0; i < kLoads; ++i) {
-            if (s == 0 && tail_here) dma_tail(wd, ad, i);
-            else dma_one(s, s, wd, ad, i);
-          }
+          for (int i = 0; i < kLoads; ++i) dma_tail(wd, ad, i);
+        } else if (s < nk) {
+#pragma unroll
+          for (int i = 0; i < kLoads; ++i) dma_one(s, s, wd, ad, i);
         }
+        if (s == 0) load_epi();
+      }
       if (nk >= STAGES) wait_vmcnt<(STAGES - 1) * kLoads>();
       else wait_vmcnt<0>();
     }
@@ -716,6 +731,7 @@ __global__ __launch_bounds__(4 * BM / FM, OCC) void gemm_big(const uint8_t* __re
     else kloop(integral_constant<int, 0>{});
     wait_vmcnt<0>();  // no DMA may still write LDS when the epilogue reuses it
   } else {
+    load_epi();
 #pragma unroll
     for (int s = 0; s < STAGES - 1; ++s) {
       if (s == 0 && tail_here) issue(s, std::true_type{});
