@@ -72,6 +72,7 @@ struct AttnArgs {
   int64_t Tk;       // cache rows (kv_index entries are clamped into it)
   int group;
   int Hkv;
+  int batches;
   int kv_len_static;
   const int32_t* kv_len;    // device kv_len or null
   const int32_t* kv_extra;  // [Tq] or null
@@ -386,6 +387,347 @@ __global__ __launch_bounds__(kAttnThreads, DT <= 4 ? 2 : 1) void attn_kernel(Att
     }
 }
 
+// ---------------------------------------------------------------------------
+// Many query rows: 64 rows per wave, software-pipelined
+// ---------------------------------------------------------------------------
+//
+// attn_kernel's waves hold 32 query rows, so every 1 KB fragment of K or V read
+// from LDS feeds one 32-cycle MFMA: at full matrix rate the four SIMDs would
+// need all of the 128 B/clk that LDS delivers, and the softmax runs beside them
+// only as far as the two workgroups of a CU happen to be out of step. Here a
+// wave holds 64 rows (two 32-row tiles), one wave per SIMD with up to 512
+// registers, and every fragment feeds two MFMAs. One iteration works on three
+// key blocks at once,
+//   S(j+1) = K(j+1) . Q^T,   O += V(j-1)^T . P(j-1),   P(j) = softmax terms of S(j),
+// which are independent of each other, so the matrix cores run under the
+// softmax arithmetic of the same wave. Rescaling of O (rare, see attn_kernel)
+// happens between iterations. K and V blocks of 64 keys come by direct-to-LDS
+// DMA into two slots each, issued at the start of an iteration for the next one,
+// with one barrier per iteration; 16-byte chunks are XOR-swizzled by row on the
+// global side so that both the row reads of K and the transposing reads of V
+// spread over all banks.
+// Measured (bf16, 24 heads of 128): 8192 tokens 1050 -> 775 us (783 -> 1065
+// TFLOP/s), 4096 tokens 327 -> 255 us. What bounds it: 2048 cycles of MFMA an
+// iteration against ~2200 of issue slots (64 exponentials at 8 cycles, 4.5
+// other vector instructions per score, 8 cycles an MFMA), which one wave per
+// SIMD cannot overlap entirely; a third slot per operand (two iterations of
+// lead for the DMA) was slower (802 us).
+template <int DT>
+struct LongTile {
+  static constexpr int kRowBytes = 64 * DT;        // one key: 32 * DT 16-bit elements
+  static constexpr int kChunks = kRowBytes / 16;   // 8 (D = 64) or 16 (D = 128)
+  static constexpr int kBytes = kBlockN * kRowBytes;
+  static constexpr int kDma = kBytes / 1024 / 4;   // DMA instructions per wave and block
+  static constexpr int kRowsPerDma = 1024 / kRowBytes;
+  // chunk position of logical chunk 0 of a row (XOR): K rows are read 16 at a
+  // time with one logical chunk, V rows 4 at a time with a pair of chunks
+  static __device__ __forceinline__ int kswz(int row) {
+    return DT == 4 ? (row & 15) : (row & 7) ^ ((row >> 3) & 1);
+  }
+  static __device__ __forceinline__ int vswz(int row) {
+    return DT == 4 ? (row & 7) << 1 : ((row >> 1) & 3) << 1;
+  }
+};
+
+template <bool BF16, int DT>
+__global__ __launch_bounds__(kAttnThreads, 1) void attn_long_kernel(AttnArgs a, int row_blocks, int per_xcd) {
+  using MF = Mfma<BF16>;
+  using T = LongTile<DT>;
+  constexpr int kC = 2 * DT;  // 16-dim chunks of the head
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[4 * T::kBytes];  // K0 K1 V0 V1
+  __shared__ int s_end[4], s_min[4];
+  uint8_t* const k_lds = lds;
+  uint8_t* const v_lds = lds + 2 * T::kBytes;
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 31;
+  const int half = lane >> 5;
+  // Workgroup b runs on XCD b % 8: each XCD walks its own contiguous range of
+  // (batch, KV head, row block), so the workgroups running on it share the K and
+  // V of one or two heads in its L2.
+  // With a causal limit the long row blocks of a head come first and alternate
+  // with short ones, so that every XCD gets the same share of keys.
+  const int logical = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  const int hb = logical / row_blocks;
+  if (hb >= a.Hkv * a.batches) return;
+  const int rbi = logical - hb * row_blocks;
+  const int rb = !a.causal ? rbi : (rbi & 1) ? rbi >> 1 : row_blocks - 1 - (rbi >> 1);
+  const int64_t b = hb / a.Hkv;
+  const int kvh = hb - static_cast<int>(b) * a.Hkv;
+
+  // this lane's two query rows
+  int64_t tok[2];
+  int head[2], lim[2];
+  bool ok[2];
+  u32x4_t qf[2][kC];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const int64_t row = static_cast<int64_t>(rb) * 256 + wave * 64 + t * 32 + col;
+    ok[t] = row < a.n_rows;
+    tok[t] = ok[t] ? row / a.group : 0;
+    head[t] = kvh * a.group + static_cast<int>(ok[t] ? row % a.group : 0);
+    const uint16_t* qp = a.q + b * a.sqb + tok[t] * a.sqt + head[t] * a.sqh + 8 * half;
+#pragma unroll
+    for (int c = 0; c < kC; ++c)
+      qf[t][c] = ok[t] ? *reinterpret_cast<const u32x4_t*>(qp + 16 * c) : u32x4_t{0u, 0u, 0u, 0u};
+  }
+  int lmax = 0, lmin = 0x7FFFFFFF;
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    lim[t] = 0;
+    if (ok[t]) {
+      lim[t] = a.kv_len ? a.kv_len[0] : a.kv_len_static;
+      if (a.kv_extra) lim[t] += a.kv_extra[tok[t]];
+      if (a.causal) lim[t] = min(lim[t], static_cast<int>(tok[t]) + a.causal_offset + 1);
+      lim[t] = max(0, min(lim[t], static_cast<int>(a.n_keys)));
+      lmin = min(lmin, lim[t]);
+    }
+    lmax = max(lmax, lim[t]);
+  }
+  {
+    const uint32_t wmax = wave_max_u32(static_cast<uint32_t>(lmax));
+    const uint32_t wmin = ~wave_max_u32(~static_cast<uint32_t>(lmin));
+    if (lane == 0) {
+      s_end[wave] = static_cast<int>(wmax);
+      s_min[wave] = static_cast<int>(wmin);
+    }
+  }
+  __syncthreads();
+  const int end = __builtin_amdgcn_readfirstlane(max(max(s_end[0], s_end[1]), max(s_end[2], s_end[3])));
+  const int full_below =
+      min(__builtin_amdgcn_readfirstlane(min(min(s_min[0], s_min[1]), min(s_min[2], s_min[3]))), end);
+  const int nb = (end + kBlockN - 1) / kBlockN;
+
+  // DMA i of this wave fills rows r0 + i * kRowsPerDma (+ lane / kChunks) of a block
+  const uint8_t* kbase = reinterpret_cast<const uint8_t*>(a.k + b * a.skb + static_cast<int64_t>(kvh) * a.skh);
+  const uint8_t* vbase = reinterpret_cast<const uint8_t*>(a.v + b * a.svb + static_cast<int64_t>(kvh) * a.svh);
+  const int64_t kstep = 2 * a.skt, vstep = 2 * a.svt;  // bytes per key
+  const int lrow = wave * T::kDma * T::kRowsPerDma + lane / T::kChunks;
+  const int lpos = lane % T::kChunks;
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_offset(lds) + wave * T::kDma * 1024);
+  auto dma_block = [&](const uint8_t* base, uint32_t step, int j, uint32_t slot, bool is_v) {
+    const int last = end - 1 - j * kBlockN;  // rows past the last visible key fetch it again
+#pragma unroll
+    for (int i = 0; i < T::kDma; ++i) {
+      const int row = lrow + i * T::kRowsPerDma;
+      const int ch = lpos ^ (is_v ? T::vswz(row) : T::kswz(row));
+      dma16s(base, __umul24(min(row, last), step) + 16 * ch, slot + i * 1024);
+    }
+  };
+  auto issue_k = [&](int j) {
+    dma_block(kbase + static_cast<int64_t>(j) * kBlockN * kstep, static_cast<uint32_t>(kstep), j,
+              lds0 + (j & 1) * T::kBytes, false);
+  };
+  auto issue_v = [&](int j) {
+    dma_block(vbase + static_cast<int64_t>(j) * kBlockN * vstep, static_cast<uint32_t>(vstep), j,
+              lds0 + (2 + (j & 1)) * T::kBytes, true);
+  };
+  auto sync = [&] {  // this wave's DMA has landed, then everybody's
+    wait_vmcnt<0>();
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): done reading the slots refilled next
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+
+  v16f acc[2][DT];
+  float m_run[2], l_run[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+#pragma unroll
+    for (int d = 0; d < DT; ++d) acc[t][d] = v16f{};
+    m_run[t] = -__builtin_inff();
+    l_run[t] = 0.0f;
+  }
+
+  auto read_k = [&](const uint8_t* kb, int kt, int c) {
+    const int row = 32 * kt + col;
+    return *reinterpret_cast<const u32x4_t*>(kb + row * T::kRowBytes + (((2 * c + half) ^ T::kswz(row)) << 4));
+  };
+  // transposing V reads as in attn_kernel: 16-lane group g, jl = lane % 16
+  const int g = lane >> 4, jl = lane & 15;
+  const int vr = 4 * (g >> 1) + (jl >> 2);
+  auto read_v = [&](const uint8_t* vb, int row0, int dt) {
+    const int row = row0 + vr;
+    const int ch = 4 * dt + 2 * (g & 1) + ((jl & 3) >> 1);
+    return lds_read_tr16(reinterpret_cast<const uint16_t*>(vb + row * T::kRowBytes + ((ch ^ T::vswz(row)) << 4) +
+                                                           8 * (jl & 1)));
+  };
+  float s[2][32];  // S of the block in work, in VGPRs (the accumulators of the next one are AccVGPRs)
+  float mb[2];     // its row maxima over this lane's keys
+  auto scores = [&](const uint8_t* kb, v16f (&sn)[2][2]) {
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) sn[t][kt] = v16f{};
+#pragma unroll
+      for (int c = 0; c < kC; ++c) {
+        const u32x4_t kf = read_k(kb, kt, c);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) sn[t][kt] = MF::run(kf, qf[t][c], sn[t][kt]);
+      }
+    }
+  };
+  float mx[2][2];
+  auto take = [&](const v16f (&sn)[2][2], int from, int to) {
+#pragma unroll
+    for (int i = from; i < to; ++i)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        s[t][i] = sn[t][i >> 4][i & 15];
+        asm volatile("" : "+v"(s[t][i]));
+        mx[t][i & 1] = i < 2 ? s[t][i] : fmaxf(mx[t][i & 1], s[t][i]);
+      }
+  };
+  constexpr int kAhead = 3, kVAhead = 2;
+
+  if (nb > 0) {
+    issue_k(0);
+    issue_v(0);
+    if (nb > 1) issue_k(1);
+    sync();
+    v16f sn[2][2];
+    scores(k_lds, sn);
+    take(sn, 0, 32);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) mb[t] = fmaxf(mx[t][0], mx[t][1]);
+  }
+  for (int j = 0; j < nb; ++j) {
+    sync();
+    if (j + 2 < nb) issue_k(j + 2);
+    if (j + 1 < nb) issue_v(j + 1);
+    const uint8_t* kb = k_lds + ((j + 1) & 1) * T::kBytes;  // past the last block: a settled slot, unused
+    const uint8_t* vb = v_lds + (j & 1) * T::kBytes;
+    const int n0 = j * kBlockN;
+    u32x4_t kf[kAhead];  // K fragments read ahead
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) kf[i] = read_k(kb, i / kC, i % kC);
+    if (n0 + kBlockN > full_below) {  // workgroup-uniform: some row does not see every key
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const int lim_b = lim[t] - n0 - 4 * half;
+        mb[t] = -__builtin_inff();
+#pragma unroll
+        for (int i = 0; i < 32; ++i) {
+          if (32 * (i >> 4) + 8 * ((i >> 2) & 3) + (i & 3) >= lim_b) s[t][i] = -__builtin_inff();
+          mb[t] = fmaxf(mb[t], s[t][i]);
+        }
+      }
+    }
+    // reference maxima (see attn_kernel), rescaling O when one moved
+    float m_use[2], alpha[2];
+    bool moved = false;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const float mx = fmaxf(mb[t], __shfl_xor(mb[t], 32, 64)) * a.qk_scale;
+      const float m_new = mx > m_run[t] + 8.0f ? fmaxf(m_run[t], mx) : m_run[t];
+      m_use[t] = m_new == -__builtin_inff() ? 0.0f : m_new;
+      alpha[t] = m_new != m_run[t] ? __builtin_amdgcn_exp2f(m_run[t] - m_use[t]) : 1.0f;
+      moved |= m_new != m_run[t];
+      m_run[t] = m_new;
+    }
+    if (__any(moved)) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        l_run[t] = l_run[t] * alpha[t];
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+          // in AccVGPRs at both ends of the rare branch: otherwise all of O is
+          // copied to VGPRs and back in every iteration
+          asm volatile("" : "+a"(acc[t][dt]));
+#pragma unroll
+          for (int i = 0; i < 16; ++i) acc[t][dt][i] = acc[t][dt][i] * alpha[t];
+          asm volatile("" : "+a"(acc[t][dt]));
+        }
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) asm volatile("" : "+a"(acc[t][dt]));
+    // The rest of the iteration is one straight line of steps of two MFMAs each,
+    // with the vector work that belongs under them and the LDS reads of a later
+    // step; sched_barrier keeps the steps apart. In order:
+    //   S(j + 1)                        under 3/4 of the exponentials of S(j)
+    //   O += V(j)^T . P(j), keys 0-31   under the last quarter
+    //   O += V(j)^T . P(j), keys 32-63  under the maxima of S(j + 1)
+    v16f sn[2][2];
+    uint32_t pk[2][2][2][4];  // P(j): [row tile][32-key tile][16-key half][packed pairs]
+    float psum[2][2] = {{0.0f, 0.0f}, {0.0f, 0.0f}};
+    auto pair = [&](int n) {  // exponentials 2n and 2n + 1 of the 64, key tile by key tile
+      const int kt = n >> 4, t = (n >> 3) & 1, i = 2 * (n & 7);
+      const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t][16 * kt + i], a.qk_scale, -m_use[t]));
+      const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t][16 * kt + i + 1], a.qk_scale, -m_use[t]));
+      psum[t][0] = psum[t][0] + p0;
+      psum[t][1] = psum[t][1] + p1;
+      pk[t][kt][i >> 3][(i & 7) >> 1] = MF::pack2(p0, p1);
+    };
+    u32x2_t vf[kVAhead][2];  // V fragments read ahead
+    auto fetch_v = [&](int i) {  // step i: key tile i / kP, 16-key half, dim tile
+      const int row0 = 16 * (i / DT);
+      vf[i % kVAhead][0] = read_v(vb, row0, i % DT);
+      vf[i % kVAhead][1] = read_v(vb, row0 + 8, i % DT);
+    };
+    constexpr int kQ = 2 * kC, kP = 2 * DT;  // steps of S, and of O per key tile
+#pragma unroll
+    for (int i = 0; i < kQ; ++i) {
+      const int kt = i / kC, c = i % kC;
+      const u32x4_t f = kf[i % kAhead];
+      if (i + kAhead < kQ) kf[i % kAhead] = read_k(kb, (i + kAhead) / kC, (i + kAhead) % kC);
+      else if (i + kVAhead >= kQ) fetch_v(i + kVAhead - kQ);
+      constexpr int kPairs = 24;
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        sn[t][kt] = MF::run(f, qf[t][c], c == 0 ? v16f{} : sn[t][kt]);
+        const int h = 2 * i + t;
+#pragma unroll
+        for (int n = h * kPairs / (2 * kQ); n < (h + 1) * kPairs / (2 * kQ); ++n) pair(n);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int i = 0; i < 2 * kP; ++i) {
+      const int kt = i / kP, qp = i / DT % 2, dt = i % DT;
+      const u32x4_t f = u32x4_t{vf[i % kVAhead][0][0], vf[i % kVAhead][0][1], vf[i % kVAhead][1][0], vf[i % kVAhead][1][1]};
+      if (i + kVAhead < 2 * kP) fetch_v(i + kVAhead);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const u32x4_t pf = u32x4_t{pk[t][kt][qp][0], pk[t][kt][qp][1], pk[t][kt][qp][2], pk[t][kt][qp][3]};
+        acc[t][dt] = MF::run(f, pf, acc[t][dt]);
+      }
+      if (kt == 0) {
+#pragma unroll
+        for (int n = 0; n < 8 / kP; ++n) pair(24 + i * (8 / kP) + n);
+      } else {
+        take(sn, (i - kP) * (32 / kP), (i - kP + 1) * (32 / kP));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      l_run[t] = l_run[t] + (psum[t][0] + psum[t][1]);
+      mb[t] = fmaxf(mx[t][0], mx[t][1]);
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const float l_tot = l_run[t] + __shfl_xor(l_run[t], 32, 64);
+    if (!ok[t]) continue;
+    const float inv = 1.0f / l_tot;
+    uint16_t* orow = a.o + b * a.sob + tok[t] * a.sot + head[t] * a.soh;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const uint32_t w0 = MF::pack2(acc[t][dt][4 * q] * inv, acc[t][dt][4 * q + 1] * inv);
+        const uint32_t w1 = MF::pack2(acc[t][dt][4 * q + 2] * inv, acc[t][dt][4 * q + 3] * inv);
+        *reinterpret_cast<u32x2_t*>(orow + 32 * dt + 8 * q + 4 * half) = u32x2_t{w0, w1};
+      }
+  }
+}
+
 // Split-KV combine for one (batch, token): merge the partial softmax states of
 // every head of the token, write O (optional) and, with q8, quantize the whole
 // token row [Hq * D] per token (this package's recipe). The per-(head, split)
@@ -511,8 +853,34 @@ void launch_attn(const AttnArgs& a, int64_t B, hipStream_t st) {
   hipLaunchKernelGGL((attn_kernel<BF16, DT>), grid, dim3(kAttnThreads), 0, st, a);
 }
 
+// Launches attn_long_kernel for the calls that it serves: see the rule inside.
+template <bool BF16>
+bool launch_long(const AttnArgs& a, int64_t B, hipStream_t st) {
+  if (a.D != 64 && a.D != 128) return false;
+  // 32-bit DMA offsets inside a block, row strides below 2^24 bytes
+  if (a.splits > 1 || a.kv_index || 2 * a.skt >= (1 << 24) || 2 * a.svt >= (1 << 24) || a.skt < 0 || a.svt < 0)
+    return false;
+  // masked scores are -inf before scaling
+  if (!(a.qk_scale > 0.0f && a.qk_scale <= 3.0e38f)) return false;
+  // Enough workgroups of 256 rows. 128 dims (MHA 1024 tokens): 64 workgroups 45.6
+  // -> 38.0 us, 96 46.9 -> 39.5, 192 58.4 -> 42.4; grouped heads, whose K and V
+  // attn_kernel finds in L2, 64 workgroups 35.2 against 38.5 us, 128 69.8 -> 66.5.
+  // 64 dims (half the matrix work per exponential): 96 workgroups 28.1 -> 27.6 us
+  // but causal 27.6 against 28.7, 144 58.7 -> 48.8.
+  const int64_t blocks = (a.n_rows + 255) / 256, total = blocks * a.Hkv * B;
+  if (total < (a.D == 64 ? 136 : a.group == 1 ? 64 : 96) || total > (1 << 28)) return false;
+  const int per_xcd = static_cast<int>((total + 7) / 8);
+  const dim3 grid(8u * per_xcd);
+  if (a.D == 128)
+    hipLaunchKernelGGL((attn_long_kernel<BF16, 4>), grid, dim3(kAttnThreads), 0, st, a, static_cast<int>(blocks), per_xcd);
+  else
+    hipLaunchKernelGGL((attn_long_kernel<BF16, 2>), grid, dim3(kAttnThreads), 0, st, a, static_cast<int>(blocks), per_xcd);
+  return true;
+}
+
 template <bool BF16>
 void dispatch_attn(const AttnArgs& a, int64_t B, int dt, hipStream_t st) {
+  if (launch_long<BF16>(a, B, st)) return;
   switch (dt) {
     case 1: launch_attn<BF16, 1>(a, B, st); break;
     case 2: launch_attn<BF16, 2>(a, B, st); break;
@@ -593,6 +961,7 @@ int ifx_attention(const void* q, const void* k, const void* v, void* o, int dtyp
   a.Tk = Tk;
   a.group = static_cast<int>(group);
   a.Hkv = static_cast<int>(Hkv);
+  a.batches = static_cast<int>(B);
   a.kv_len_static = static_cast<int>(kv_len < a.n_keys ? kv_len : a.n_keys);
   a.kv_len = kv_len_dev;
   a.kv_extra = kv_extra;

@@ -36,6 +36,14 @@ def _close(out, ref, dtype, what=""):
     assert err < BAR[dtype], f"{what} max |d| {err:.3e}"
 
 
+def _close_rounded(out, ref, dtype, what):
+    # rows of few keys reach |out| ~ 4, where rounding the output alone takes up to 2^-8 (bf16) or 2^-11
+    # (fp16) of it; the bar above is what the rounded probabilities may add
+    err = np.abs(out.float().cpu().numpy() - ref)
+    u = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    assert (err <= BAR[dtype] + u * np.abs(ref)).all(), f"{what} max |d| {err.max():.3e}"
+
+
 @pytest.mark.parametrize("hd,hq,hkv", [(256, 8, 1), (72, 16, 16), (128, 16, 2)])
 def test_dynamic_length(gpu, oracle_mod, hd, hq, hkv):
     # tests/test_gi_kernels.py:32-41
@@ -101,6 +109,47 @@ def test_shapes_bf16(gpu, oracle_mod, B, Tq, Tk, hq, hkv, hd, splits):
     ws = SplitWorkspace(B, Tq, hq, hkv, hd, splits, gpu) if splits > 1 else None
     out = attention(q.to(gpu), k.to(gpu), v.to(gpu), split=ws)
     _close(out, _ref(oracle_mod, q, k, v, np.full(Tq, Tk)), torch.bfloat16, f"B{B} Tq{Tq} Tk{Tk} hd{hd}")
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,Tq,Tk,hq,hkv,hd,opts", [
+    (8, 40, 1, 16, 16, 128, {}), (8, 70, 64, 16, 16, 128, {}),          # one key, one whole block, a short row block
+    (4, 300, 65, 16, 16, 128, dict(kv_len=50)), (9, 33, 127, 16, 16, 64, {}),
+    (2, 1100, 300, 8, 8, 128, {}), (5, 257, 200, 24, 24, 64, dict(kv_len=131)),
+    (6, 40, 300, 32, 16, 128, dict(extra=True)),                         # grouped heads
+    (1, 1000, 1000, 16, 16, 128, dict(causal=0)), (3, 700, 750, 16, 16, 64, dict(causal=50)),
+    (4, 300, 320, 16, 16, 128, dict(causal=-20, scale=0.2))])            # rows without a visible key
+def test_many_rows(gpu, oracle_mod, dtype, B, Tq, Tk, hq, hkv, hd, opts):
+    # enough 256-row workgroups for the 64-rows-per-wave kernel; operands are strided views of one buffer
+    from instinctflash_amd.kernels import attention
+    q, k, v = _qkv(B, Tq, Tk, hq, hkv, hd, Tq + Tk, dtype)
+    kv = torch.zeros(B, Tk, 2, hkv, hd, dtype=dtype, device=gpu)
+    kv[:, :, 0], kv[:, :, 1] = k.to(gpu), v.to(gpu)
+    kw, lim = {}, np.full(Tq, Tk)
+    if "kv_len" in opts:
+        kw["kv_len"] = torch.tensor([opts["kv_len"]], device=gpu, dtype=torch.int32)
+        lim = np.full(Tq, opts["kv_len"])
+    if opts.get("extra"):
+        extra = torch.arange(Tq, dtype=torch.int32)
+        kw.update(kv_len=Tk - Tq, kv_extra=extra.to(gpu), max_extra=Tq)
+        lim = Tk - Tq + np.arange(Tq)
+    if "causal" in opts:
+        kw.update(causal=True, causal_offset=opts["causal"])
+        lim = np.clip(np.arange(Tq) + opts["causal"] + 1, 0, Tk)
+    out = attention(q.to(gpu), kv[:, :, 0], kv[:, :, 1], scale=opts.get("scale"), **kw)
+    see = lim > 0  # a row without keys has no defined result
+    ref = _ref(oracle_mod, q[:, see], k, v, lim[see], scale=opts.get("scale"))
+    _close_rounded(out[:, torch.from_numpy(see)], ref, dtype, f"{B}x{Tq}x{Tk} {hq}/{hkv}x{hd}")
+
+
+def test_many_rows_moving_maximum(gpu, oracle_mod):
+    # scores that grow along the keys by far more than the 2^8 the reference maximum may lag: O is rescaled in
+    # many iterations, differently per row
+    from instinctflash_amd.kernels import attention
+    q, k, v = _qkv(8, 64, 600, 16, 16, 128, 5, torch.bfloat16)
+    k = (k * torch.linspace(0.1, 12, 600)[None, :, None, None]).to(torch.bfloat16)
+    out = attention(q.to(gpu), k.to(gpu), v.to(gpu))
+    _close_rounded(out, _ref(oracle_mod, q, k, v, np.full(64, 600)), torch.bfloat16, "moving maximum")
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
