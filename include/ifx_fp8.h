@@ -187,11 +187,11 @@ int ifx_dequant_rows(const void* x, int x_dtype, int64_t ldx, int64_t M, int64_t
  * lda/ldw multiples of 16, ldo/ldr multiples of 8. sa: f32 [M] or NULL,
  * sw: f32 [N] or NULL, bias: f32 [N] or NULL, gate: bf16 [N_out] or NULL.
  * workspace: at least ifx_fp8_linear_workspace_size(M,N,K,epilogue) bytes of
- * 16-byte aligned device memory, used when the GEMM (M > 64) splits K across
+ * 16-byte aligned device memory, used when the GEMM (M > 16) splits K across
  * workgroups because it has too few output tiles to fill the GPU: the slices'
  * fp32 partial sums, added by a second launch. The size is 0 (NULL allowed)
- * otherwise, and always for M <= 64. With K % 128 != 0 a smaller workspace (or
- * NULL) is accepted too: K is then not split. No initialisation is needed; one
+ * otherwise. With K % 128 != 0 or M <= 64 a smaller workspace (or NULL) is
+ * accepted too: K is then not split. No initialisation is needed; one
  * workspace serves any sequence of calls and shapes. Calls that may overlap
  * must not share a workspace.
  * With sa = sw = NULL and epilogue 0 this is the raw-accumulator GEMM of
@@ -331,8 +331,8 @@ int ifx_wan_qkv(const void* raw, int raw_dtype, int64_t ldraw, const float* row,
  * IFX_SCALE_TENSOR needs ldx == K (else IFX_ERR_UNSUPPORTED).
  * workspace: ifx_quant_linear_workspace_size(...) bytes, 256-byte aligned, no
  * initialisation needed; calls that may overlap must not share one. With
- * K % 128 != 0 the part of ifx_fp8_linear_workspace_size may be missing (K is
- * then not split).
+ * K % 128 != 0 or M <= 64 the part of ifx_fp8_linear_workspace_size may be
+ * missing (K is then not split).
  * a_scale: NULL, or [M] f32 (IFX_SCALE_ROW) / [1] f32 (IFX_SCALE_TENSOR) that
  * receives the activation scales. IFX_EPI_SCALAR_SA is rejected (the scale is
  * computed here); IFX_EPI_SCALAR_SW is honoured.
@@ -421,7 +421,8 @@ int ifx_attention(const void* q, const void* k, const void* v, void* o, int dtyp
  * call on that GPU until the process ends). No allocation of any kind.
  * Rejects with IFX_ERR_SCRATCH a call whose ifx_quant_linear_workspace_size
  * exceeds the scratch (about M * K bytes of e4m3 plus the split-K partials;
- * with K % 128 != 0 a call whose partials do not fit runs without a split).
+ * with K % 128 != 0 or M <= 64 a call whose partials do not fit runs without
+ * a split).
  * The scratch is looked up on the CURRENT device (hipGetDevice), which must be
  * the device of `stream` and of every operand. All calls on one GPU share its
  * scratch: calls that may overlap on one GPU (distinct streams without

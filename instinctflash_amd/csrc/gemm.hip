@@ -22,11 +22,11 @@
 // unchanged.
 //
 // Kernels (dispatch in ifx_fp8_linear)
-//  * gemm_big (M > 64): 256 weight rows x 256 (or fewer) tokens
+//  * gemm_big (M > 64, and many weight rows or a long K from M = 17 on): 256 weight rows x 256 (or fewer) tokens
 //    per workgroup, 32x32x64 MFMAs, operands copied global -> LDS by
 //    direct-to-LDS DMA through a multi-stage ring, LDS-staged epilogue; split K
 //    (+ splitk_reduce) when the output has too few tiles to fill the GPU.
-//  * gemm_skinny (M <= 64): bound by the weight stream. A workgroup owns 16 (32
+//  * gemm_skinny (other M <= 64): bound by the weight stream. A workgroup owns 16 (32
 //    for GLU) weight rows and the whole of K; its waves split the K steps,
 //    stream weight fragments straight from HBM into MFMA registers, and add
 //    their partial sums in LDS in a fixed order (deterministic).
@@ -334,7 +334,10 @@ __device__ __forceinline__ v4f quad(const v16f& v, int q) {
 // What a DMA lane fetches for a chunk past K.
 __device__ const uint8_t kZeroChunk[16] __attribute__((aligned(16))) = {};
 
-template <int BM, int BN, int KB, int STAGES, int OCC, bool GLU, int FM>
+// TL: an operand may be in the tile layout of ifx_fp8_pack_skinny (as the
+// epilogue flags say); a variant of its own, because the choice of the layout
+// per DMA costs the small tiles 1%.
+template <int BM, int BN, int KB, int STAGES, int OCC, bool GLU, int FM, bool TL>
 __global__ __launch_bounds__(4 * BM / FM, OCC) void gemm_big(const uint8_t* __restrict__ A, int64_t lda,
                                                      const uint8_t* __restrict__ W, int64_t ldw, int64_t K,
                                                      TileMap tmap, Epi e, Partials part) {
@@ -433,25 +436,37 @@ __global__ __launch_bounds__(4 * BM / FM, OCC) void gemm_big(const uint8_t* __re
   const int lpos = lane % S::kChunks;
   const uint32_t lds_base = __builtin_amdgcn_readfirstlane(lds_offset(smem) + wave * kLoads * 1024);
   const int64_t n_last = e.N - 1, m_last = e.M - 1;
+  const bool w_tiled = TL && (e.flags & IFX_EPI_W_TILED), a_tiled = TL && (e.flags & IFX_EPI_A_TILED);
+  const int64_t tile_rows = (K + kBK - 1) / kBK * 2048;  // bytes of 16 rows in the tile layout
+  // chunk `ch` of row `row`, `k` bytes from the first stage; the tile layout's
+  // stages lie 2048 bytes apart
+  auto tiled_off = [=](int64_t row, int ch, int64_t k) {
+    return (row >> 4) * tile_rows + (row & 15) * 16 + (ch & 1) * 1024 + (ch >> 1) * 256 + k * (2048 / KB);
+  };
   // Issues this wave's DMAs of local stage kl (K stage kt0 + kl) into ring slot
   // kl % STAGES; with the tag, of the partial stage, whose chunks past K come
   // from zeros.
   auto issue = [&](int kl, auto tail_tag) {
     constexpr bool kTail = decltype(tail_tag)::value;
     const uint32_t buf = lds_base + (kl % STAGES) * kStage;
+    const int64_t k0 = kTail ? K - tail : static_cast<int64_t>(kt0 + kl) * KB - kshift;
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) {
       const int blk = wave * kLoads + i;
       const int row = blk * kRowsPerDma + lrow;
-      const int kb = (lpos ^ S::f(row)) << 4;
-      const int64_t k0 = (kTail ? K - tail : static_cast<int64_t>(kt0 + kl) * KB - kshift) + kb;
+      const int ch = lpos ^ S::f(row);
+      const int64_t k = k0 + (ch << 4);
       const uint8_t* p;
       if (blk * kRowsPerDma < BN) {  // wave-uniform
-        p = W + min(n0 + row, n_last) * ldw + k0;
+        const int64_t n = min(n0 + row, n_last);
+        if (w_tiled) p = W + tiled_off(n, ch, k0);
+        else p = W + n * ldw + k;
       } else {
-        p = A + min(m0 + (row - BN), m_last) * lda + k0;
+        const int64_t m = min(m0 + (row - BN), m_last);
+        if (a_tiled) p = A + tiled_off(m, ch, k0);
+        else p = A + m * lda + k;
       }
-      if constexpr (kTail) p = kb < tail ? p : kZeroChunk;
+      if constexpr (kTail) p = ch * 16 < tail ? p : kZeroChunk;
       dma16(p, buf + i * 1024);
     }
   };
@@ -1459,12 +1474,13 @@ struct BigPlan {
   int64_t kstages;  // K stages per slice
 };
 
-inline BigPlan big_plan(int64_t M, int64_t N, int64_t K, bool may_split) {
+inline BigPlan big_plan(int64_t M, int64_t N, int64_t K, bool may_split, double* us = nullptr) {
   const int64_t nk = (K + kBK - 1) / kBK;
   const int64_t most = may_split ? max_split(M, N, nk) : 1;
   BigPlan best{};
   double best_t = 0;
-  for (int i = 0; i < static_cast<int>(std::size(kBigCost)); ++i) {
+  // up to 64 tokens: the tiles that read the tile layouts
+  for (int i = M <= kSkinnyMaxM ? static_cast<int>(BigCfg::kSmall) : 0; i < static_cast<int>(std::size(kBigCost)); ++i) {
     const BigCost& c = kBigCost[i];
     const int64_t tiles = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
     for (int64_t s = 1; s <= most && (s == 1 || tiles * s <= 512); ++s) {
@@ -1477,6 +1493,7 @@ inline BigPlan big_plan(int64_t M, int64_t N, int64_t K, bool may_split) {
       }
     }
   }
+  if (us) *us = best_t;
   return best;
 }
 
@@ -1487,19 +1504,19 @@ inline size_t split_bytes(int64_t M, int64_t N, int64_t K) {
 }
 
 // Whether a call may run without the workspace its K split wants: a K that is
-// no multiple of 128 needed none before such shapes were split, so a caller
-// without it (a stream being captured, a fixed scratch buffer) is still served,
-// by unsplit tiles.
-inline bool split_optional(int64_t K) { return K % kBK != 0; }
+// no multiple of 128, or up to 64 tokens, needed none before such shapes were
+// split, so a caller without it (a stream being captured, a fixed scratch
+// buffer) is still served, by unsplit tiles or the skinny kernel.
+inline bool split_optional(int64_t M, int64_t K) { return M <= kSkinnyMaxM || K % kBK != 0; }
 
-template <int BM, int BN, int KB, int STAGES, int OCC, bool GLU, int FM = 2>
+template <int BM, int BN, int KB, int STAGES, int OCC, bool GLU, int FM = 2, bool TL = false>
 int launch_big(const uint8_t* a, int64_t lda, const uint8_t* w, int64_t ldw, int64_t K, const Epi& e,
                void* ws, const BigPlan& p, hipStream_t st) {
   const int64_t tiles_m = (e.M + BM - 1) / BM, tiles_n = (e.N + BN - 1) / BN;
   if (tiles_m * tiles_n * p.ksplit > 0x7FFFFFF0LL) return IFX_ERR_UNSUPPORTED;
   const Partials part{p.ksplit > 1 ? static_cast<float*>(ws) : nullptr, e.N, p.kstages};
   const TileMap t = make_tile_map(tiles_m, tiles_n, p.ksplit);
-  hipLaunchKernelGGL((gemm_big<BM, BN, KB, STAGES, OCC, GLU, FM>), dim3(static_cast<unsigned>(8 * t.per_xcd)), dim3(4 * BM / FM),
+  hipLaunchKernelGGL((gemm_big<BM, BN, KB, STAGES, OCC, GLU, FM, TL>), dim3(static_cast<unsigned>(8 * t.per_xcd)), dim3(4 * BM / FM),
                      0, st, a, lda, w, ldw, K, t, e, part);
   if (p.ksplit > 1) {
     const int64_t threads = e.M * ((GLU ? e.N / 2 : e.N) / 4);
@@ -1517,14 +1534,45 @@ inline bool dma32_ok(int64_t M, int64_t N, int64_t lda, int64_t ldw) {
   return M < k24 && N < k24 && lda < k24 && ldw < k24 && M * lda < k32 && N * ldw < k32;
 }
 
+// Whether 17 to 64 tokens take gemm_big's 32- and 64-token tiles instead of the
+// skinny kernel. The skinny kernel reads the activations again for every 16 (GLU:
+// 32) weight rows, straight from L2 into registers; with many weight rows or a
+// long K that stream is what it waits for. In gemm_big a workgroup shares them
+// among 128 weight rows through LDS. Measured with weights streamed from HBM,
+// skinny / gemm_big, us:
+//   row-major: 51x34176x768 31.1 / 12.1, 64x8192x8192 44.5 / 20.2, 64x2048x16384
+//     37.4 / 14.0, 48x16384x1024 14.0 / 8.3, 20x32768x1024 17.3 / 9.2; but
+//     64x8192x1024 9.6 / 7.9, 64x4096x2048 9.4 / 10.7, 32x8192x4096 17.0 / 12.6
+//   tile layouts: 64x32768x1024 18.6 / 10.7, 20x32768x1024 11.8 / 9.7, 64x16384x4096
+//     28.6 / 23.0, 48x8192x8192 24.1 / 20.5; but 48x16384x1024 9.2 / 9.4,
+//     64x16384x2048 GeGLU 12.4 / 13.7, 64x8192x4096 15.3 / 22.0
+// For the tile layouts the lines are these measurements. Row-major weights also
+// take it where its fitted cost (or its weights at 5 TB/s) beats by 3 us the
+// skinny kernel's stream at 7.3 TB/s and 3 ns per row group past one per CU;
+// around that line both take the same.
+inline bool small_path(int64_t M, int64_t N, int64_t K, int epilogue) {
+  if (M <= 16) return false;
+  const bool glu = (epilogue & (IFX_EPI_GEGLU | IFX_EPI_SWIGLU)) != 0;
+  const double mb = static_cast<double>((M + 15) / 16), weights = static_cast<double>(N) * K;
+  // bytes the skinny kernel's workgroups read (see skinny_plan's token split)
+  const double stream = weights * (glu ? 1 + mb / 2 : N < 4096 ? 2 * mb : 1 + mb);
+  if (N >= 32768 || (M > 48 && N >= 16384 && (!glu || K <= 1024)) || (!glu && stream >= 190e6)) return true;
+  if (epilogue & IFX_EPI_W_TILED) return false;
+  double us = 0;
+  big_plan(M, N, K, true, &us);
+  const double groups = static_cast<double>(N) / (glu ? 32 : 16);
+  return std::max(us, 4.0 + weights / 5.0e6) + 3.0 < 2.0 + stream / 7.3e6 + (groups > 256 ? 3e-3 * groups : 0.0);
+}
+
 template <bool GLU>
 int launch_large(const uint8_t* a, int64_t lda, const uint8_t* w, int64_t ldw, int64_t K, const Epi& e, void* ws,
                  size_t ws_bytes, hipStream_t st) {
   const size_t need = split_bytes(e.M, e.N, K);
   const bool have = need == 0 || (ws && ws_bytes >= need && aligned16(ws));
-  if (!have && !split_optional(K)) return IFX_ERR_WORKSPACE;
+  if (!have && !split_optional(e.M, K)) return IFX_ERR_WORKSPACE;
   const BigPlan p = big_plan(e.M, e.N, K, have);
   const bool dma32 = dma32_ok(e.M, e.N, lda, ldw);
+  const bool tiled = (e.flags & (IFX_EPI_W_TILED | IFX_EPI_A_TILED)) != 0;  // M <= 64: one of the small tiles
   switch (p.cfg) {
     case BigCfg::kWide192:
       if (dma32) return launch_big<256, 192, 128, 2, 1, GLU, 4>(a, lda, w, ldw, K, e, ws, p, st);
@@ -1533,8 +1581,12 @@ int launch_large(const uint8_t* a, int64_t lda, const uint8_t* w, int64_t ldw, i
     case BigCfg::kWide:
       if (dma32) return launch_big<256, 256, 128, 2, 1, GLU, 4>(a, lda, w, ldw, K, e, ws, p, st);
       return launch_big<256, 256, 128, 2, 1, GLU>(a, lda, w, ldw, K, e, ws, p, st);
-    case BigCfg::kSmall: return launch_big<64, 128, 128, 3, 2, GLU, 1>(a, lda, w, ldw, K, e, ws, p, st);
-    case BigCfg::kSmall32: return launch_big<32, 128, 128, 3, 2, GLU, 1>(a, lda, w, ldw, K, e, ws, p, st);
+    case BigCfg::kSmall:
+      if (tiled) return launch_big<64, 128, 128, 3, 2, GLU, 1, true>(a, lda, w, ldw, K, e, ws, p, st);
+      return launch_big<64, 128, 128, 3, 2, GLU, 1>(a, lda, w, ldw, K, e, ws, p, st);
+    case BigCfg::kSmall32:
+      if (tiled) return launch_big<32, 128, 128, 3, 2, GLU, 1, true>(a, lda, w, ldw, K, e, ws, p, st);
+      return launch_big<32, 128, 128, 3, 2, GLU, 1>(a, lda, w, ldw, K, e, ws, p, st);
     case BigCfg::kNarrow192:
       if (dma32) return launch_big<128, 192, 128, 3, 1, GLU, 2>(a, lda, w, ldw, K, e, ws, p, st);
       [[fallthrough]];
@@ -1552,9 +1604,8 @@ using namespace ifx;
 extern "C" {
 
 size_t ifx_fp8_linear_workspace_size(int64_t M, int64_t N, int64_t K, int epilogue) {
-  (void)epilogue;  // every epilogue of a shape takes the same slices
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  if (M <= kSkinnyMaxM) return 0;  // the skinny kernel needs no workspace
+  if (M <= kSkinnyMaxM && !small_path(M, N, K, epilogue)) return 0;  // the skinny kernel needs none
   return split_bytes(M, N, K);
 }
 
@@ -1642,7 +1693,10 @@ int ifx_fp8_linear(const void* a, int64_t lda, const float* sa, const void* w, i
   const uint8_t* Wt = static_cast<const uint8_t*>(w);
   hipStream_t st = static_cast<hipStream_t>(stream);
 
-  if (M <= kSkinnyMaxM) {
+  // (a shape whose split wants a workspace that the caller does not have: skinny)
+  const size_t split_ws = split_bytes(M, N, K);
+  if (M <= kSkinnyMaxM && (!small_path(M, N, K, epilogue) ||
+                           (split_ws > 0 && (!workspace || ws_bytes < split_ws || !aligned16(workspace))))) {
     const SkinnyPlan p = skinny_plan(M, N, K, glu);
     return glu ? launch_skinny<2>(p, A, lda, Wt, ldw, K, e, st) : launch_skinny<1>(p, A, lda, Wt, ldw, K, e, st);
   }
@@ -1743,7 +1797,7 @@ int ifx_quant_linear(const void* x, int64_t ldx, int scale_mode, const void* w, 
   if (rc != IFX_OK || M == 0) return rc;
   // the stand-alone quantizer into the workspace, then the GEMM
   QlWorkspace ql = ql_workspace(M, N, K, epilogue, scale_mode);
-  if (ws_bytes < ql.total && split_optional(K)) ql = ql_workspace(M, N, K, epilogue, scale_mode, false);
+  if (ws_bytes < ql.total && split_optional(M, K)) ql = ql_workspace(M, N, K, epilogue, scale_mode, false);
   if (!workspace || ws_bytes < ql.total || (reinterpret_cast<uintptr_t>(workspace) & 255u)) return IFX_ERR_WORKSPACE;
   uint8_t* base = static_cast<uint8_t*>(workspace);
   void* gws = base;
@@ -1825,7 +1879,7 @@ int ifx_quant_linear_noalloc(const void* x, int64_t ldx, int scale_mode, const v
   // every contract check before the scratch is touched: a rejected call launches nothing
   int rc = check_quant_linear(x, ldx, scale_mode, w, ldw, sw, bias, residual, ldr, gate, epilogue, out, ldo, M, N, K);
   if (rc != IFX_OK || M == 0) return rc;
-  const size_t need = ql_workspace(M, N, K, epilogue, scale_mode, !split_optional(K)).total;
+  const size_t need = ql_workspace(M, N, K, epilogue, scale_mode, !split_optional(M, K)).total;
   if (need > kScratchBytes) return IFX_ERR_SCRATCH;
   void* ws = scratch_ptr(&rc);
   if (!ws) return rc;

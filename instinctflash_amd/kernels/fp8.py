@@ -135,7 +135,7 @@ _WORKSPACES: dict = {}
 _RETIRED: list = []
 
 
-def _workspace(nbytes: int, device, stream: int, least: int | None = None):
+def _workspace(nbytes: int, device, stream: int, optional: int = 0):
     """(buffer, usable bytes) of the workspace per (device, stream), reused by every call on that stream
     (calls on one stream are ordered). It holds split-K partial sums, which
     every call writes before it reads them, so it needs no initialisation.
@@ -143,8 +143,8 @@ def _workspace(nbytes: int, device, stream: int, least: int | None = None):
     A buffer outgrown by a later call is kept alive (never freed), because a
     captured HIP graph may still hold its address. Growing while the stream is
     being captured raises instead: run the captured calls once eagerly first,
-    so the buffer is already large enough. A call that can also run with
-    ``least`` bytes (without its K split) takes what there is under capture."""
+    so the buffer is already large enough. A call that can also run without
+    ``optional`` of its bytes (its K split) takes what there is under capture."""
     if nbytes == 0:
         return None, 0
     key = (device.index, stream)
@@ -152,7 +152,7 @@ def _workspace(nbytes: int, device, stream: int, least: int | None = None):
     if ws is None or ws.numel() < nbytes:
         if torch.cuda.is_current_stream_capturing():
             have = 0 if ws is None else ws.numel()
-            if least is not None and have >= least:
+            if optional and have >= nbytes - optional:
                 return ws, have
             raise RuntimeError(f"the FP8 workspace of this stream must grow to {nbytes} bytes during HIP graph "
                                "capture; run the captured calls once before capturing")
@@ -358,7 +358,7 @@ def _linear(a, sa, w: Fp8Weight, out, flags, residual=None, gate=None, use_scale
     lib = _lib.load()
     stream = _stream(a.device)
     nbytes = lib.ifx_fp8_linear_workspace_size(M, N, K, flags)
-    ws, nbytes = _workspace(nbytes, a.device, stream, 0 if K % 128 else None)
+    ws, nbytes = _workspace(nbytes, a.device, stream, nbytes if K % 128 or M <= 64 else 0)
     _lib.check(lib.ifx_fp8_linear(_ptr(a_t), lda, _ptr(sa) if use_scales else None, _ptr(w.w), ldw,
                                   _ptr(sw), _ptr(bias), _ptr(residual), ldr, _ptr(gate), flags,
                                   _ptr(out), ldo, M, N, K, _ptr(ws), nbytes, stream), "ifx_fp8_linear")
@@ -428,8 +428,10 @@ def quant_linear(x: torch.Tensor, w: Fp8Weight, out: torch.Tensor | None = None,
     lib = _lib.load()
     stream = _stream(x.device)
     nbytes = lib.ifx_quant_linear_workspace_size(M, N, K, flags, mode)
-    least = nbytes - -(-lib.ifx_fp8_linear_workspace_size(M, N, K, flags) // 256) * 256 if K % 128 else None
-    ws, nbytes = _workspace(nbytes, x.device, stream, least)
+    optional = 0
+    if (K % 128 or M <= 64) and torch.cuda.is_current_stream_capturing():
+        optional = -(-lib.ifx_fp8_linear_workspace_size(M, N, K, flags) // 256) * 256
+    ws, nbytes = _workspace(nbytes, x.device, stream, optional)
     _lib.check(lib.ifx_quant_linear(_ptr(x), ldx, mode, _ptr(w.w), ldw, _ptr(sw), _ptr(bias), _ptr(residual), ldr,
                                     _ptr(gate), flags, _ptr(out), ldo, M, N, K, _ptr(a_scale), _ptr(ws), nbytes,
                                     stream), "ifx_quant_linear")

@@ -135,7 +135,7 @@ def linear_qkv_rope(a, a_scale, w, q_out, k_out, v_out, *, inv_freq=None, pos=No
     rows ``kv_base + t``. Replaces ``gemm`` + ``qkv_split`` (reference
     kernels/fp8.py:50-53, kernels/rope.py:89-116) without the bf16 round trip of
     the raw accumulator; no per-head norms, no position sections."""
-    from .fp8 import TiledRows, E4M3, _workspace
+    from .fp8 import TiledRows, E4M3
     if w.rope is None:
         raise ValueError("linear_qkv_rope needs a weight from permute_rope_rows")
     HQ, HKV, HD = w.rope
@@ -188,11 +188,9 @@ def linear_qkv_rope(a, a_scale, w, q_out, k_out, v_out, *, inv_freq=None, pos=No
         return q_out
     lib = _lib.load()
     stream = _stream(dev)
-    nbytes = lib.ifx_fp8_linear_workspace_size(M, N, K, 0)
-    ws, nbytes = _workspace(nbytes, dev, stream)
     _lib.check(lib.ifx_fp8_linear_qkv_rope(
         _ptr(a_t), lda, _ptr(a_scale), _ptr(w.w), ldw, _ptr(w.scale), _ptr(w.bias), flags,
         _ptr(pos) if inv_freq is not None else None, ldpos, _ptr(inv_freq), HQ, HKV, HD,
         _ptr(q_out), sq[0], sq[1], _ptr(k_out), sk[0], sk[1], _ptr(v_out), sv[0], sv[1], _OUT[q_out.dtype],
-        base_rows, _ptr(kv_base) if dynamic else None, M, K, _ptr(ws), nbytes, stream), "ifx_fp8_linear_qkv_rope")
+        base_rows, _ptr(kv_base) if dynamic else None, M, K, None, 0, stream), "ifx_fp8_linear_qkv_rope")
     return q_out

@@ -477,6 +477,44 @@ def test_skinny_token_block_forms(gpu, oracle_mod, M, N, K, act):
     assert torch.equal(got.view(torch.int32), o32.view(torch.int32)), f"tiled skinny blocks {M}x{N}x{K}"
 
 
+@pytest.mark.parametrize("M,N,K,act", [
+    (17, 32784, 272, None), (51, 34176, 768, "gelu_tanh"), (33, 32800, 144, "geglu"),  # unsplit, ragged N and K
+    (64, 16384, 528, "swiglu"), (49, 16400, 128, None),
+    (51, 768, 17088, None), (64, 2048, 16400, None), (40, 3072, 12288, "gelu_tanh")])  # split K
+def test_few_tokens_shared_tiles(gpu, oracle_mod, M, N, K, act):
+    # 17-64 tokens with many weight rows or a long K: the 32- and 64-token tiles, from row-major and from tile
+    # layouts (every pairing of the two operands, bit-identical: the same bytes reach the same fragments; only
+    # the row-major weight of 51 x 768 x 17088 takes these tiles)
+    from instinctflash_amd.kernels import TiledRows, fp8 as F, pack_glu, pack_skinny, quant_rows_tiled
+    glu = act in ("geglu", "swiglu")
+    qa, sa, fw, g = _make(gpu, M, N, K, seed=M + N + K, bias=True)
+    res = torch.randn((M, N // 2 if glu else N), generator=g).to(torch.bfloat16)
+    w = pack_glu(fw) if glu else fw
+    o32, _ = _check(gpu, oracle_mod, qa, sa, w, f"few {M}x{N}x{K}", ref_w=fw, act=act, residual=res)
+    tiles = torch.from_numpy(_tile_rows_np(_q(qa), M, K)).to(gpu).view(torch.float8_e4m3fn).reshape(-1)
+    for a in (qa, TiledRows(tiles, M, K)):
+        for weight in (w,) if N == 768 else (w, pack_skinny(w)):
+            got = F.linear(a, sa, weight, act=act, residual=res.to(gpu), out_dtype=torch.float32)
+            assert torch.equal(got.view(torch.int32), o32.view(torch.int32)), f"{M}x{N}x{K} {type(a)} {weight.tiled}"
+
+
+def test_few_tokens_without_workspace(gpu, oracle_mod):
+    # up to 64 tokens need no workspace: captured on a stream that has none, the call takes the skinny kernel
+    from instinctflash_amd.kernels import linear
+    M, N, K = 51, 768, 17088
+    qa, sa, fw, _ = _make(gpu, M, N, K, seed=12, bias=True)
+    out = torch.empty((M, N), device=gpu)
+    linear(qa, sa, fw, out=out)
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.graph(graph, stream=side):
+        linear(qa, sa, fw, out=out)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        _assert_close(_f(out), _ref(oracle_mod, qa, sa, fw), "no workspace")
+
+
 @pytest.mark.parametrize("M,N,K", [(16, 1536, 6144), (16, 768, 3072), (8, 1024, 4096), (1, 1024, 16384),
                                    (16, 512, 8192)])
 def test_skinny_needs_no_workspace(gpu, M, N, K):
