@@ -70,6 +70,12 @@ def test_wan5b_shape(gpu, oracle_mod, out_dtype):
     _run_check(gpu, oracle_mod, 2, 64, 24, 128, True, True, out_dtype, 1)
 
 
+@pytest.mark.parametrize("out_dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T", [1820, 1821])  # below and above 32 MB of 16-bit outputs at 24 x 128
+def test_large_outputs(gpu, oracle_mod, out_dtype, T):
+    _run_check(gpu, oracle_mod, 1, T, 24, 128, True, True, out_dtype, seed=T)
+
+
 @pytest.mark.parametrize("H,HD", [(4, 64), (8, 256), (2, 8), (40, 128), (48, 256)])
 def test_shapes(gpu, oracle_mod, H, HD):
     _run_check(gpu, oracle_mod, 1, 33, H, HD, True, True, torch.bfloat16, H + HD)
