@@ -186,6 +186,21 @@ def test_per_tensor_quant(gpu, oracle_mod, shape, mag):
     _nan_eq_bytes(_q(q), eq)
 
 
+@pytest.mark.parametrize("count", [8, 8184, 8192, 8200, 131072, 131080])
+def test_per_tensor_one_launch_edges(gpu, oracle_mod, count):
+    # up to 16 chunks of 8192 elements in one launch, two launches above; the largest value in the last group
+    from instinctflash_amd.kernels import quantize_tensor
+    x = torch.randn(count, generator=torch.Generator().manual_seed(count)).to(torch.bfloat16)
+    x[-1] = -37.0
+    q, s = quantize_tensor(x.to(gpu))
+    eq, es = oracle_mod.quant_tensor(_bits(x))
+    assert _f(s).view(np.uint32)[0] == es.view(np.uint32)[0]
+    _nan_eq_bytes(_q(q), eq)
+    x[count // 2] = float("nan")
+    q, s = quantize_tensor(x.to(gpu))
+    assert torch.isnan(s).all() and ((_q(q) & 0x7F) == 0x7F).all()
+
+
 def test_per_tensor_all_patterns_and_nan(gpu, oracle_mod):
     from instinctflash_amd.kernels import quantize_tensor
     x = all_finite_bf16().reshape(1, -1)
