@@ -116,6 +116,8 @@ class IfxError(RuntimeError):
 def load(path: Path | str | None = None) -> ctypes.CDLL:
     """Load (once) and return the library; raise if it is missing or its ABI differs."""
     global _lib
+    if path is None and _lib is not None:  # set once, after every signature is declared
+        return _lib
     with _lock:
         if _lib is not None and path is None:
             return _lib
