@@ -391,7 +391,7 @@ int dispatch_rows(const Src& src, bool vec_ok, int64_t M, int64_t K, uint8_t* q,
   return launch_status();
 }
 
-// ---- per-tensor quantizer (two launches, no host sync) --------------------
+// ---- per-tensor quantizer (one or two launches, no host sync) --------------------
 
 constexpr int64_t kTensorChunk = 8192;  // elements per partial (one block)
 
@@ -491,8 +491,8 @@ __global__ __launch_bounds__(kBlock) void tensor_pack_vec(const uint16_t* x, int
 // kTensorChunk, one group per lane. A per-tensor quant_linear (this and a
 // GEMM) replayed in a graph, two quantizer launches -> one: 1024 elements 6.83 ->
 // 5.31 us, 24576 8.83 -> 6.67, 51200 11.74 -> 9.78, 131072 14.74 -> 13.78.
-// Larger tensors keep the two launches: the reads
-// repeated per block grow with the square of the size.
+// Larger tensors keep the two launches: the reads repeated per block grow with the
+// square of the size.
 constexpr int kOneLanes = kTensorChunk / 8;
 constexpr int64_t kTensorOneMax = 16 * kTensorChunk;
 
